@@ -28,6 +28,19 @@ __device__ __forceinline__ half8 as_half8(u32x4 u) {
   return h;
 }
 
+// Eight biased int8 weights (two words) as halves, exactly: byte b (= q + 128) under 0x64 is the half 1024 + b.
+__device__ __forceinline__ half8 i8x8_to_half8(uint32_t w0, uint32_t w1) {
+  const uint32_t k64 = 0x64646464u;
+  const uint32_t a0 = __builtin_amdgcn_perm(k64, w0, 0x04010400u);
+  const uint32_t a1 = __builtin_amdgcn_perm(k64, w0, 0x04030402u);
+  const uint32_t a2 = __builtin_amdgcn_perm(k64, w1, 0x04010400u);
+  const uint32_t a3 = __builtin_amdgcn_perm(k64, w1, 0x04030402u);
+  u32x4 u = {a0, a1, a2, a3};
+  half8 h = as_half8(u);
+  const half8 bias = {1152, 1152, 1152, 1152, 1152, 1152, 1152, 1152};
+  return h - bias;
+}
+
 template <typename T>
 __device__ __forceinline__ T ldg(const T* p) {
   typedef __attribute__((address_space(1))) const T GT;

@@ -302,6 +302,20 @@ int gemm_launch(GemmParams& p, bool i8, hipStream_t s);
 // order of the int8-x products (LFM3_X8), piece-major within a lane's 16 bytes.
 int gemm_tile_launch(const void* src, void* dst, int N, int K, hipStream_t s, int x8 = 0);
 
+// Many-token GEMM on int8 weights (gemm_wide.hip): y[band][n][N] = the band's share of scale * x q^T.
+struct GemmWideParams {
+  const _Float16* x;       // [n][K] row-major
+  const uint8_t* w;        // the tile-major copy of [N][K] biased int8 (gemm_tile_launch, x8 = 0)
+  const _Float16* scale;   // [N], or
+  const _Float16* gscale;  // [K / 128][N]
+  float* y;                // [bands][n][N]
+  int n, N, K;
+  int tile, bands, band_chunks;  // gemm_wide_plan: rows and tokens of a tile, shares of K and their 64-column chunks
+};
+// false: a shape this kernel does not take (N % 128, operands of 2 GiB or more)
+bool gemm_wide_plan(int n, int N, int K, bool gs, int max_bands, GemmWideParams* p);
+int gemm_wide_launch(const GemmWideParams& p, hipStream_t s);
+
 size_t verify_argmax_ws(int M, int V);
 
 // fold = false: the partial keys [M][verify_argmax_chunks(V)] stay in ws for accept_commit_fold_launch to fold.

@@ -106,6 +106,10 @@ struct dspark_engine {
   // State per projection chunk (ctx_pos, ctx_new of the chunk)
   _Float16* tapx = nullptr;
   int tap_rows = 0, tap_from = -1;
+  // whole-prompt projection (project_wide): the GEMM outputs of up to tap_rows positions (fc's two bands, then ckv's
+  // rows) and the hidden norm's x
+  float* proj_y = nullptr;
+  _Float16* proj_x = nullptr;
   dspark_state* seed_st = nullptr;
   int seed_chunks = 0;
   std::vector<dspark_state> host_seed;
@@ -507,6 +511,49 @@ int enqueue_context(dspark_engine* e, const _Float16* x_fc, bool x_op, hipStream
   return 0;
 }
 
+// The context projection of n prompt positions at once, x_fc row-major [n][n_taps * H]: the same four steps as
+// enqueue_context, each one launch over every position, its GEMMs (planned by project_wide_plan) on many-token tiles (gemm_wide.hip).
+constexpr int PROJ_BANDS = 2;  // proj_y holds tap_rows x PROJ_BANDS x H: fewer positions may take more bands
+bool project_wide_plan(dspark_engine* e, int n, GemmWideParams* fc, GemmWideParams* ckv) {
+  const dspark_model_desc& d = e->d;
+  const bool gs = d.weight_format == 1;
+  return gemm_wide_plan(n, d.hidden, d.n_taps * d.hidden, gs, PROJ_BANDS * e->tap_rows / n, fc) &&
+         gemm_wide_plan(n, d.draft_layers * 2 * d.kv_heads * d.head_dim, d.hidden, gs, 1, ckv);
+}
+int project_wide(dspark_engine* e, const _Float16* x_fc, int n, GemmWideParams fc, GemmWideParams ckv, hipStream_t s) {
+  const dspark_model_desc& d = e->d;
+  const int H = d.hidden, kvrow = 2 * d.kv_heads * d.head_dim, rows = d.draft_layers * kvrow;
+  const bool gs = d.weight_format == 1;
+  auto gemm_of = [&](GemmWideParams& p, const _Float16* x, const uint8_t* w, const _Float16* sc) {
+    p.x = x;
+    p.w = e->tiles[e->tile_of[w]].dst;
+    (gs ? p.gscale : p.scale) = sc;
+    p.y = e->proj_y;
+    return gemm_wide_launch(p, s);
+  };
+  CK(gemm_of(fc, x_fc, e->fc_w, e->fc_s));
+  ResNormParams p = {};
+  p.st = e->ast;
+  p.v = e->proj_y;
+  p.bands = fc.bands;
+  p.v_band_stride = (size_t)n * H;
+  p.norm_w = e->hidden_norm;
+  p.eps = d.eps;
+  p.x16 = e->proj_x;
+  p.x_row = H;
+  p.H = H;
+  CK(resnorm_launch(p, n, 1, s));
+  CK(gemm_of(ckv, e->proj_x, e->ckv_w, e->ckv_s));
+  for (int j0 = 0; j0 < d.draft_layers; j0 += QKROPE_BATCH) {
+    QkRopeBatch b = {};
+    b.n = std::min(QKROPE_BATCH, d.draft_layers - j0);
+    for (int j = 0; j < b.n; ++j)
+      b.l[j] = qk_params(e, e->DL[j0 + j], e->proj_y + (size_t)(j0 + j) * kvrow, rows, false, true, n);
+    CK(qkrope_batch_launch(b, s));
+  }
+  return 0;
+}
+
 // The round's launch sequence (see the file header). mv: verify width, the token rows of the verify pass (the
 // round's drafts are capped below it, so 1 + drafts <= mv; the drafter block stays B wide). skip: a skip round
 // (dspark.hip:2441-2451): the context projection, then the anchor alone verified (no drafter), State.skip decremented.
@@ -853,6 +900,10 @@ int dspark_engine_create(const dspark_model_desc* desc, int32_t max_context, dsp
   // GEMM reads), one State per chunk of B positions
   e->tap_rows = (d.draft_window + B - 1) / B * B + B;
   e->tapx = h16("tap_x", (size_t)e->tap_rows * d.n_taps * H);
+  if (d.x_format == 0) {
+    e->proj_y = static_cast<float*>(e->alloc("", (size_t)e->tap_rows * std::max(PROJ_BANDS * H, ckv_rows) * 4, &err));
+    e->proj_x = static_cast<_Float16*>(e->alloc("", (size_t)e->tap_rows * H * 2, &err));
+  }
   e->seed_chunks = e->tap_rows / B;
   e->seed_st = static_cast<dspark_state*>(e->alloc("", (size_t)e->seed_chunks * sizeof(dspark_state), &err));
   // request state and activations
@@ -1158,20 +1209,30 @@ int dspark_engine_project_prompt(dspark_engine* e, int32_t first, int32_t end, d
     const int rc = prepare(e, s, false);
     if (rc) return rc;
   }
-  const int B = e->B, nch = (end - first + B - 1) / B;
+  // Every position in one pass where that pays: beyond one block of positions the chunks below run the same four
+  // launches per block, each latency-bound (2048 positions: 3.13 ms in 128 chunks). x_format 1 keeps the chunks (its
+  // GEMMs quantize x per 16 columns as they load it).
+  const int B = e->B;
+  GemmWideParams fc = {}, ckv = {};
+  const bool wide = e->d.x_format == 0 && end - first > B && project_wide_plan(e, end - first, &fc, &ckv);
+  const int nch = wide ? 1 : (end - first + B - 1) / B;
   if (nch > e->seed_chunks) return DSPARK_EINVAL;
   e->host_seed.assign(nch, dspark_state{});
   for (int c = 0; c < nch; ++c) {
     dspark_state& t = e->host_seed[c];
     t.run = 1;
     t.ctx_pos = first + c * B;
-    t.ctx_new = std::min(B, end - t.ctx_pos);
+    t.ctx_new = wide ? end - first : std::min(B, end - t.ctx_pos);
   }
   if (hipMemcpyAsync(e->seed_st, e->host_seed.data(), nch * sizeof(dspark_state), hipMemcpyHostToDevice, s) != hipSuccess)
     return DSPARK_EINVAL;
   const size_t row = (size_t)e->d.n_taps * e->d.hidden;
   int rc = 0;
-  for (int c = 0; c < nch && !rc; ++c) {
+  if (wide) {
+    e->ast = e->seed_st;
+    rc = project_wide(e, e->tapx, end - first, fc, ckv, s);
+  }
+  for (int c = 0; c < nch && !rc && !wide; ++c) {
     e->ast = e->seed_st + c;
     rc = enqueue_context(e, e->tapx + (size_t)c * B * row, false, s);
   }

@@ -18,18 +18,6 @@
 
 namespace dspark {
 
-__device__ __forceinline__ half8 i8x8_to_half8(uint32_t w0, uint32_t w1) {
-  const uint32_t k64 = 0x64646464u;
-  const uint32_t a0 = __builtin_amdgcn_perm(k64, w0, 0x04010400u);
-  const uint32_t a1 = __builtin_amdgcn_perm(k64, w0, 0x04030402u);
-  const uint32_t a2 = __builtin_amdgcn_perm(k64, w1, 0x04010400u);
-  const uint32_t a3 = __builtin_amdgcn_perm(k64, w1, 0x04030402u);
-  u32x4 u = {a0, a1, a2, a3};
-  half8 h = as_half8(u);
-  const half8 bias = {1152, 1152, 1152, 1152, 1152, 1152, 1152, 1152};
-  return h - bias;
-}
-
 __device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
 
 // Epilogue for one lane's 4 rows (row0 + 4g + i) of token t.

@@ -1,0 +1,68 @@
+"""The drafter's prompt projection over many positions in one pass (dspark_engine_project_prompt past one block):
+captured taps -> fc -> hidden norm -> ckv -> k norm + RoPE -> ring rows, on the many-token GEMM's two tile sizes with row
+and group scales, at position counts around the tiles' edges, against fp64 from the same weights.
+
+Bar: the ring holds fp16 of values whose inputs the GPU and the check round to fp16 at the same points (the captured taps,
+the hidden norm's output), so a value differs by its own rounding and by what last-bit flips of those inputs carry
+through a dot product: two fp16 steps at the largest magnitude, the bar of the blockwise projection's test."""
+import numpy as np
+import pytest
+
+from conftest import load_host, rope_numpy
+from test_gpu_engine import REF_SMALL, SMALL, make_weights
+from test_gpu_launch import ulp16
+
+pytestmark = pytest.mark.gpu
+
+# 64-token tiles, K in bands (2 taps x 256 columns: 8 chunks), 2 drafter layers
+NARROW = dict(SMALL, draft_window=700, ring_positions=1024)
+# group scales, head_dim 128
+GROUPS = dict(REF_SMALL, draft_window=700, ring_positions=1024, weight_format=1)
+# 128-token tiles for fc (16 x 13 tiles at 1537 positions), 64-token ones for ckv, an odd number of chunks per band
+WIDE = dict(SMALL, hidden=2048, q_heads=32, kv_heads=8, ffn=256, draft_ffn=256, n_taps=1, tap_layer=[1],
+            draft_window=1600, ring_positions=2048)
+WIDE_GROUPS = dict(WIDE, weight_format=1, n_taps=3, tap_layer=[0, 1, 2])
+CASES = [(NARROW, n, first) for n, first in ((9, 0), (63, 5), (64, 31), (65, 7), (128, 0), (200, 500), (700, 330))]
+CASES += [(GROUPS, n, 33) for n in (10, 64, 129, 511)]
+CASES += [(WIDE, 1537, 700), (WIDE_GROUPS, 1537, 1), (WIDE_GROUPS, 1600, 0)]
+
+
+@pytest.mark.parametrize("geom,n,first", CASES)
+def test_many_positions(geom, n, first):
+    import torch
+    from oracle import round as rnd
+    host = load_host()
+    desc = host.model_desc(**geom)
+    H, KVH, D = desc.hidden, desc.kv_heads, desc.head_dim
+    print(f"case hidden={H} n={n} first={first} weight_format={desc.weight_format}", flush=True)
+    eng = host.Engine(desc, 2560)
+    W = rnd.Weights(desc, make_weights(eng, desc, 7))
+    rng = np.random.default_rng(n)
+    taps = rng.standard_normal((desc.n_taps, n, H)).astype(np.float16)
+    for slot in range(desc.n_taps):
+        eng.capture_tap(slot, torch.from_numpy(taps[slot]).cuda(), first, first)
+    eng.project_prompt(first, first + n)
+    torch.cuda.synchronize()
+
+    x = np.concatenate([rnd.tap_rows(W, taps[b].astype(np.float64), b) for b in range(desc.n_taps)], axis=1)
+    c = rnd.gemm(x, *W.gemm_w("fc", H, desc.n_taps * H))
+    _, x = rnd.resnorm(None, c, None, W.f16("hidden_norm"), 0, desc.eps)
+    kv = rnd.gemm(x, *W.gemm_w("ckv", desc.draft_layers * 2 * KVH * D, H)).reshape(n, desc.draft_layers, 2, KVH, D)
+    rope = rnd.h2f(rope_numpy(desc.rope_base, desc.rope_pairs, D, first + n))[first:][:, None, :]
+    cos, sin, half, p = rope[..., :D // 2], rope[..., D // 2:], D // 2, desc.rope_pairs
+    bt = torch.from_numpy(eng.download("ring_table", np.int32))
+    for j in range(desc.draft_layers):
+        k = kv[:, j, 0]
+        k = k / np.sqrt((k * k).mean(-1, keepdims=True) + desc.eps) * W.f16(f"D{j}.k_norm")
+        wk = k.copy()
+        wk[..., :p] = k[..., :p] * cos[..., :p] - k[..., half:half + p] * sin[..., :p]
+        wk[..., half:half + p] = k[..., half:half + p] * cos[..., :p] + k[..., :p] * sin[..., :p]
+        kp = torch.from_numpy(eng.download(f"ring.D{j}.k", np.uint16)).view(torch.float16).reshape(-1, KVH, 32, D)
+        vp = torch.from_numpy(eng.download(f"ring.D{j}.v", np.uint16)).view(torch.float16).reshape(-1, KVH, D, 32)
+        gk, gv = (a.astype(np.float64) for a in host.kv_from_pages(kp, vp, range(first, first + n), bt))
+        kerr, verr = np.max(np.abs(gk - wk)), np.max(np.abs(gv - kv[:, j, 1]))
+        print(f"layer {j}: K max-abs {kerr:.2e}, V max-abs {verr:.2e}", flush=True)
+        assert kerr <= 2 * ulp16(np.max(np.abs(wk))) and verr <= 2 * ulp16(np.max(np.abs(kv[:, j, 1])))
+        outside, _ = host.kv_from_pages(kp, vp, [first + n] + ([first - 1] if first else []), bt)
+        assert not np.any(outside)
+    eng.close()
