@@ -488,7 +488,7 @@ __device__ __forceinline__ void gscale_products(f32x4& acc, const u32x2 (&gsr)[C
 // piece: lane (g, n) gives row n's / token n's columns 16 p + 4 g .. + 3 of piece p. The weight tiles of an int8-x
 // engine are laid out for it (gemm_tile_kernel, x8: byte b of lane (g, n) is column 16 (b / 4) + 4 g + b % 4 of the
 // 64-column chunk, so a[p / 2] halves 4 (p % 2) .. + 3 are piece p's four weights); row-major weights (the C ABI) are
-// gathered in the same order. Codes are integer-valued halves, so each product is the piece's exact integer dot
+// brought to the same order (x8_transpose4). Codes are integer-valued halves, so each product is the piece's exact integer dot
 // (|dot| <= 16 * 127 * 127 < 2^24). p.x8 = 1: x is fp16 and each piece is quantized by the four lanes that hold it, as
 // x_fill does (883-904): s = max(max|x| / 127, 1e-20), codes rint(x * rcp(s)); p.x8 = 2: x holds the codes (the norm
 // kernel's output) and p.xsc the scales [token][K / 16].
@@ -525,29 +525,42 @@ __device__ __forceinline__ uint32_t pmax_u16_lanes(uint32_t v) {
   return pmax_u16(b[0], b[1]);
 }
 
-// p.x8 == 1: quantize the lane's 4 pieces (each piece's 16 values sit in the lanes (g', n), g' = 0..3); returns the
-// piece scales and turns xq into codes. max|x| is taken on the fp16 bit patterns, two pieces per packed word.
-__device__ __forceinline__ f32x4 x8_quantize(u32x2 (&xq)[4]) {
-  uint32_t pm[4];
+// The 4 x 4 transpose of dwords over the lanes n, n + 16, n + 32, n + 48: out[j] of lane group g = v[g] of lane group j
+// (two half-wave swaps each of the VALU, no LDS).
+__device__ __forceinline__ u32x4 x8_transpose4(u32x4 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return u32x4{c[0], c[1], d[0], d[1]};
+}
+
+// p.x8 == 1: quantize piece g of a chunk, whole in lane (n, g) (lo: its columns 0 .. 7, hi: 8 .. 15); returns its scale
+// and turns lo and hi into codes. max|x| is taken on the fp16 bit patterns.
+__device__ __forceinline__ float x8_quantize_piece(u32x4& lo, u32x4& hi) {
+  const u32x4 m4 = {pmax_u16(lo[0] & 0x7fff7fffu, hi[0] & 0x7fff7fffu), pmax_u16(lo[1] & 0x7fff7fffu, hi[1] & 0x7fff7fffu),
+                    pmax_u16(lo[2] & 0x7fff7fffu, hi[2] & 0x7fff7fffu), pmax_u16(lo[3] & 0x7fff7fffu, hi[3] & 0x7fff7fffu)};
+  const uint32_t m2 = pmax_u16(pmax_u16(m4[0], m4[1]), pmax_u16(m4[2], m4[3]));
+  const float s = x8_piece_scale(x8_mag_value(max(m2 & 0xffffu, m2 >> 16)));
+  const float inv = __builtin_amdgcn_rcpf(s);
+  half8 a = as_half8(lo), b = as_half8(hi);
 #pragma unroll
-  for (int pc = 0; pc < 4; ++pc) pm[pc] = pmax_u16(xq[pc][0] & 0x7fff7fffu, xq[pc][1] & 0x7fff7fffu);
-  uint32_t m2[2];  // pieces 2 k (low half) and 2 k + 1 (high half)
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    m2[k] = pmax_u16_lanes(pmax_u16(__builtin_amdgcn_perm(pm[2 * k + 1], pm[2 * k], 0x05040100u),
-                                    __builtin_amdgcn_perm(pm[2 * k + 1], pm[2 * k], 0x07060302u)));
-  f32x4 sc;
-#pragma unroll
-  for (int pc = 0; pc < 4; ++pc) {
-    half4v h = __builtin_bit_cast(half4v, xq[pc]);
-    const float s = x8_piece_scale(x8_mag_value((m2[pc >> 1] >> (16 * (pc & 1))) & 0xffffu));
-    const float inv = __builtin_amdgcn_rcpf(s);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) h[j] = (_Float16)rintf((float)h[j] * inv);
-    xq[pc] = __builtin_bit_cast(u32x2, h);
-    sc[pc] = s;
+  for (int j = 0; j < 8; ++j) {
+    a[j] = x8_code(a[j], inv);
+    b[j] = x8_code(b[j], inv);
   }
-  return sc;
+  lo = __builtin_bit_cast(u32x4, a);
+  hi = __builtin_bit_cast(u32x4, b);
+  return s;
+}
+// The chunk's 4 pieces in the products' order (xq[p] of lane (n, g): columns 4 g .. 4 g + 3 of piece p) and their scales,
+// from raw x with piece g whole in lane (n, g).
+__device__ __forceinline__ f32x4 x8_quantize(u32x4 lo, u32x4 hi, u32x2 (&xq)[4]) {
+  const uint32_t s = __builtin_bit_cast(uint32_t, x8_quantize_piece(lo, hi));
+  const u32x4 even = x8_transpose4(u32x4{lo[0], lo[2], hi[0], hi[2]}), odd = x8_transpose4(u32x4{lo[1], lo[3], hi[1], hi[3]});
+#pragma unroll
+  for (int pc = 0; pc < 4; ++pc) xq[pc] = u32x2{even[pc], odd[pc]};
+  return __builtin_bit_cast(f32x4, x8_transpose4(u32x4{s, s, s, s}));
 }
 
 // One chunk under LFM3_X8: accg[r] += dot_p[r] * xs[p] over its 4 pieces (accg: the 128-column group's sum, scaled by
@@ -595,8 +608,9 @@ __device__ __forceinline__ f32x4 x8_scales_load(const GemmParams& p, int n, int 
 }
 
 // X8: 0 fp16 x; 1 int8 x quantized as it is loaded (p.x8 == 1); 2 int8 codes + scales given (p.x8 == 2).
-// TO (int8 x): tile-major weights only -- with the row-major form also compiled in, whose chunk is four loads against
-// one, the compiler cannot count a batch's loads past the layout test and waits for all of them before the first product.
+// TO (int8 x): tile-major weights; else row-major ones, loaded 16 bytes a lane as everywhere and put in the products'
+// order in registers. (Gathered there as four dword loads each fetched 16 of every 64 bytes: 15360 x 2048 at 8 tokens
+// @A@, 2048 x 7680 @B@.)
 template <int TB, bool I8, int CPW, bool XD, int MAXT = 1024, bool GS = false, int X8 = 0, bool ONEB = false,
           bool TO = false>
 __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
@@ -638,7 +652,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
 #pragma unroll
   for (int tb = 0; tb < TB; ++tb) acc[tb] = f32x4{0, 0, 0, 0};
 
-  const bool tiled = I8 && (TO || p.tiled);
+  const bool tiled = X8 ? TO : I8 && p.tiled;
   const uint8_t* wrow = tiled ? reinterpret_cast<const uint8_t*>(p.w) + (size_t)strip * chunks * 1024 + lane * 16
                               : reinterpret_cast<const uint8_t*>(p.w) + (size_t)(row0 + n) * p.K * (I8 ? 1 : 2) + 16 * g;
   const int cstride = tiled ? 1024 : 64;
@@ -648,12 +662,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
 #pragma unroll
     for (int i = 0; i < CPW; ++i) {
       const int c = min(cb + i, max(c1, 1) - 1);
-      if (X8 && !tiled) {
-        // row-major weights in the int8-x tile order: byte b = column 16 (b / 4) + 4 g + b % 4 of the chunk
-        const uint8_t* rp = reinterpret_cast<const uint8_t*>(p.w) + (size_t)(row0 + n) * p.K + (size_t)c * 64 + 4 * g;
-        w[i][0] = u32x4{ldg_nt(reinterpret_cast<const uint32_t*>(rp)), ldg_nt(reinterpret_cast<const uint32_t*>(rp + 16)),
-                        ldg_nt(reinterpret_cast<const uint32_t*>(rp + 32)), ldg_nt(reinterpret_cast<const uint32_t*>(rp + 48))};
-      } else if (I8) {
+      if (I8) {
         w[i][0] = ldg_nt(reinterpret_cast<const u32x4*>(wrow + (size_t)c * cstride));
       } else {
         const u32x4* wp = reinterpret_cast<const u32x4*>(wrow + 2 * c * 64 + 16 * g);
@@ -662,13 +671,15 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
       }
     }
   };
-  auto weights = [&](const u32x4 (&w)[WV], half8 (&a)[2]) {
+  auto weights = [&](const u32x4 (&wr)[WV], half8 (&a)[2]) {
+    // (row-major weights under int8 x: lane (n, g)'s 16 bytes are piece g; the tiles hold the products' order)
+    const u32x4 w0 = X8 && !TO ? x8_transpose4(wr[0]) : wr[0];
     if (I8) {
-      a[0] = i8x8_to_half8(w[0][0], w[0][1]);
-      a[1] = i8x8_to_half8(w[0][2], w[0][3]);
+      a[0] = i8x8_to_half8(w0[0], w0[1]);
+      a[1] = i8x8_to_half8(w0[2], w0[3]);
     } else {
-      a[0] = as_half8(w[0]);
-      a[1] = as_half8(w[WV - 1]);
+      a[0] = as_half8(w0);
+      a[1] = as_half8(wr[WV - 1]);
     }
   };
   u32x4 w[CPW][WV];
@@ -682,19 +693,19 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     // compiler's wait for the previous iteration's loads would also hold the first batch back behind the flag load.
     // Token block tb of chunk c (operand order, TB > 1 needs it): the next 1 KB block pair, tb * 1024 halves on.
     auto batch = [&](int cb) {
-      u32x4 xb[X8 ? 1 : CPW][TB][2];
-      u32x2 xq[X8 ? CPW : 1][4];
+      u32x4 xb[X8 == 2 ? 1 : CPW][TB][2];
+      u32x2 xq[X8 == 2 ? CPW : 1][4];
       u32x2 gsr[GS ? CPW / 2 : 1];
-      f32x4 xsl[X8 ? CPW : 1];
+      f32x4 xsl[X8 == 2 ? CPW : 1];
 #pragma unroll
       for (int i = 0; i < CPW; ++i) {
         const int c = min(cb + i, c1 - 1);
-        if constexpr (X8) {
+        if constexpr (X8 == 2) {
           const X8Src xsrc = x8_src(p, g, n);
 #pragma unroll
           for (int pc = 0; pc < 4; ++pc)
             xq[i][pc] = ldg(reinterpret_cast<const u32x2*>(xsrc.base + (size_t)c * xsrc.cstride + pc * xsrc.pstride));
-          if (X8 == 2) xsl[i] = x8_scales_load(p, n, c);
+          xsl[i] = x8_scales_load(p, n, c);
         } else {
 #pragma unroll
           for (int tb = 0; tb < TB; ++tb) {
@@ -715,8 +726,12 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
           if (cb + i < c1) {
             half8 a[2];
             weights(w[i], a);
-            const f32x4 xs4 = X8 == 2 ? xsl[i] : x8_quantize(xq[i]);
-            x8_chunk(accg, a, xq[i], xs4);
+            if constexpr (X8 == 2) {
+              x8_chunk(accg, a, xq[i], xsl[i]);
+            } else {
+              const f32x4 xs4 = x8_quantize(xb[i][0][0], xb[i][0][1], xq[0]);
+              x8_chunk(accg, a, xq[0], xs4);
+            }
           }
           // a 128-column group ends after its second chunk (or the range's last): scale it by the rows' group scales
           if ((i & 1) && cb + i - 1 < c1) {
@@ -783,10 +798,10 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
       }
     };
     u32x2 gsr[GS ? CPW / 2 : 1];
-    // LFM3_X8 codes from the norm (p.x8 == 2): the band's piece scales go to LDS after its X^T, [chunk][token] x 16 B
-    // (token t's 4 pieces of the chunk), by the same kind of loads (issued before the weights, so the counted wait
-    // below covers them)
-    const f32x4* xsc_lds = reinterpret_cast<const f32x4*>(xs + (size_t)(b1 - b0) * 2 * 64);
+    // LFM3_X8: the band's piece scales go to LDS after its X^T, [chunk][token] x 16 B (token t's 4 pieces of the chunk).
+    // Codes from the norm (p.x8 == 2): by the same kind of loads (issued before the weights, so the counted wait below
+    // covers them).
+    f32x4* xsc_lds = reinterpret_cast<f32x4*>(xs + (size_t)(b1 - b0) * 2 * 64);
     if constexpr (X8 == 2) {
       {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -806,6 +821,20 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     load(w, c0);
     __builtin_amdgcn_s_waitcnt(GEMM_VMCNT(CPW * WV));
     __builtin_amdgcn_s_barrier();
+    if constexpr (X8 == 1) {
+      // x quantized where it lies, each chunk once in the workgroup (lane (n, g): token n's piece g): the products below
+      // then read codes and scales as the norm would have left them. (Quantized by each of the strips' waves as they
+      // read it: @C@.)
+      for (int j = wave_u; j < bc; j += nw) {
+        u32x4* xr = xs + (size_t)j * 2 * 64 + lane;
+        u32x4 lo = xr[0], hi = xr[64];
+        reinterpret_cast<float*>(xsc_lds + (size_t)(j >> 2) * 64 + 16 * (j & 3) + n)[g] = x8_quantize_piece(lo, hi);
+        xr[0] = lo;
+        xr[64] = hi;
+      }
+      __builtin_amdgcn_s_waitcnt(GEMM_LGKMCNT0);  // (the weights stay in flight)
+      __builtin_amdgcn_s_barrier();
+    }
     if constexpr (X8) {  // one token block, X^T of the band in LDS at once, as below
       for (int cb = c0; cb < c1; cb += CPW) {
         if (cb != c0) {
@@ -827,8 +856,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
               xq[pc] = *reinterpret_cast<const u32x2*>(xb + (((g >> 1) * 64 + 16 * pc + n) * 16 + 8 * (g & 1)));
             // chunk j's scales of token n: 4-chunk rows of 64 lanes, row (j - b0) / 4, lane 16 ((j - b0) % 4) + n
             const int jr = cb + i - b0;
-            const f32x4 xs4 = X8 == 2 ? xsc_lds[(jr >> 2) * 64 + 16 * (jr & 3) + n] : x8_quantize(xq);
-            x8_chunk(accg, a, xq, xs4);
+            x8_chunk(accg, a, xq, xsc_lds[(jr >> 2) * 64 + 16 * (jr & 3) + n]);
           }
           if ((i & 1) && cb + i - 1 < c1) {
             const half4 ws = __builtin_bit_cast(half4, gsr[i >> 1]);
@@ -1049,13 +1077,16 @@ static bool gemm_sliced_xd(const GemmParams& p, bool i8) {
   return i8 && p.xd && (p.M <= 16 || (p.xop && p.M <= 64 && p.wpg * p.kw <= 8 && !p.gscale));
 }
 
+// LDS of a band's int8-x piece scales, after its X^T.
+static size_t gemm_x8_scale_bytes(int band_chunks) { return (size_t)(band_chunks + 3) / 4 * 1024; }
+
 // LDS of a K-sliced launch: X^T (unless each wave loads its own), the range sums, the fused epilogue's tile.
 static size_t gemm_sliced_lds_bytes(const GemmParams& p, bool i8) {
   const int tb = (p.M + 15) / 16;
   const int bands = std::max(1, p.bands);
   const int bc = (p.K / 64 + bands - 1) / bands;  // X^T of the token blocks of one pass (all of them when they fit)
   size_t x = gemm_sliced_xd(p, i8) ? 0 : (size_t)gemm_pass_tbs(tb, bc) * bc * 2048;
-  if (x && p.x8 == 2) x += (size_t)(bc + 3) / 4 * 1024;  // the band's int8-x piece scales after X^T
+  if (x && p.x8) x += gemm_x8_scale_bytes(bc);
   const size_t red = (size_t)(p.kw - 1) * p.wpg * tb * 1024;
   const size_t tile = p.fuse ? (size_t)tb * 16 * (16 * p.wpg + 4) * sizeof(float) : 0;
   const size_t ex = p.ysc && p.epilogue == 1 ? (size_t)16 * p.wpg * sizeof(uint32_t) : 0;  // gemm_gated_x8_out
@@ -1328,10 +1359,13 @@ int gemm_launch(GemmParams& p, bool i8, hipStream_t s) {
     // K-sliced: whole K in one workgroup of wpg x kw <= 16 waves; X^T in LDS (<= 64 KB) unless one strip per group
     const int tb = (p.M + 15) / 16;
     if (p.bands < 1) p.bands = 1;
-    if (p.ksplit != 1 || p.wpg < 1 || p.wpg * p.kw > 16 || tb > 4 || gemm_sliced_lds_bytes(p, i8) > GEMM_X_LDS)
+    const int bc = (p.K / 64 + p.bands - 1) / p.bands;
+    // (x quantized in LDS: its scales come on top of an X^T that may fill the limit by itself)
+    if (p.ksplit != 1 || p.wpg < 1 || p.wpg * p.kw > 16 || tb > 4 ||
+        gemm_sliced_lds_bytes(p, i8) > GEMM_X_LDS + (p.x8 == 1 ? gemm_x8_scale_bytes(bc) : 0))
       return DSPARK_EINVAL;
     // X^T in passes (it does not fit LDS for every token block at once): each range within one batch of weights
-    const int bc = (p.K / 64 + p.bands - 1) / p.bands, cpk = (bc + p.kw - 1) / p.kw;
+    const int cpk = (bc + p.kw - 1) / p.kw;
     const int tp = gemm_pass_tbs(tb, bc);
     if (!gemm_sliced_xd(p, i8) && ((size_t)tp * bc * 2048 > GEMM_X_LDS || (tp < tb && cpk > 8) || (tb > 2 && cpk > 8)))
       return DSPARK_EINVAL;
