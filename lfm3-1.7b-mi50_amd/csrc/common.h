@@ -59,6 +59,18 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 __device__ __forceinline__ constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 constexpr int LGKMCNT0_IMM = 0xC07F;
 
+// A ring step's hand-over: this wave's direct-to-LDS loads but the N youngest done, and its reads of the step before (whose
+// slot the loads issued next overwrite), then every wave's. The wait and barrier builtins do not order memory operations
+// for the compiler, which sees no other writer of the slot read next: the empty asm holds every access on its side, and the
+// LDS count is waited for because the uses of the last step's reads may sink below.
+template <int N>
+__device__ __forceinline__ void ring_barrier() {
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(N) & ~0x0F00);  // lgkmcnt(0) too
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));

@@ -98,8 +98,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(GemmWideParams p) {
   // x piece q = 2 g + h of the lane's token (rows 16 tb + n; the slot's rows start at a multiple of 8 tokens)
   const int xq0 = n * 128 + (((2 * g) ^ (n & 7)) * 16), xq1 = n * 128 + (((2 * g + 1) ^ (n & 7)) * 16);
   auto step = [&](int k, const char* cur, char* nxt) {
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPW));
-    __builtin_amdgcn_s_barrier();  // chunk k is in LDS; every wave is done with chunk k - 1 (its slot is nxt)
+    ring_barrier<LPW>();  // chunk k is in LDS; every wave is done with chunk k - 1 (its slot is nxt)
     issue(min(k + 2, nc - 1), nxt);
     half8 a[SR][2];
     half4 gs[GS ? SR : 1];  // (read every step: under the branch below the compiler would drain every load first)
