@@ -95,6 +95,21 @@ AttnParams attn_params(const dspark_attn_args* a) {
   return p;
 }
 
+// What the streamed GEMM's 16-byte loads into LDS need of the caller's operands.
+bool on_16_bytes(const void* x, const void* w) {
+  return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+}
+
+void gemm_take_plan(GemmParams& p, const GemmPlan& pl) {
+  p.ksplit = pl.ksplit;
+  p.wpg = pl.wpg;
+  p.cpb = pl.cpb;
+  p.kw = pl.kw;
+  p.xd = pl.xd;
+  p.stream = pl.stream;
+  p.few = pl.few;
+}
+
 }  // namespace
 
 extern "C" {
@@ -302,7 +317,7 @@ int dspark_accept_commit(dspark_state* st, const uint64_t* best_keys, int32_t M,
 
 size_t dspark_gemm_i8_workspace(int32_t M, int32_t N, int32_t K) {
   if (M < 1 || M > 64 || N < 16 || N % 16 || K < 64 || K % 64) return 0;
-  return gemm_ws_bytes(M, N, K);
+  return std::max(gemm_ws_bytes(M, N, K), gemm_ws_bytes(M, N, K, 0, false, true));  // whichever way the operands lie
 }
 
 int dspark_gemm_i8(const void* x, int32_t M, int32_t K, const uint8_t* w, const void* scale, int32_t N,
@@ -323,12 +338,8 @@ int dspark_gemm_i8(const void* x, int32_t M, int32_t K, const uint8_t* w, const 
   p.K = K;
   p.epilogue = epilogue;
   GemmPlan pl;
-  gemm_plan(M, N, K, true, true, &pl);
-  p.ksplit = pl.ksplit;
-  p.wpg = pl.wpg;
-  p.cpb = pl.cpb;
-  p.kw = pl.kw;
-  p.xd = pl.xd;
+  gemm_plan(M, N, K, true, true, &pl, 0, false, 1, false, on_16_bytes(x, w));
+  gemm_take_plan(p, pl);
   if (p.ksplit > 1) {
     if (gemm_groups(pl, N) > GEMM_COUNTER_SLOTS) return DSPARK_EINVAL;
     if (!workspace || workspace_bytes < gemm_ws_bytes(pl, M, N)) return DSPARK_ENOSPACE;
@@ -355,12 +366,8 @@ int dspark_gemm_i8_g128(const void* x, int32_t M, int32_t K, const uint8_t* w, c
   p.K = K;
   p.epilogue = epilogue;
   GemmPlan pl;
-  gemm_plan(M, N, K, true, false, &pl, 0, false, 1, true);
-  p.ksplit = pl.ksplit;
-  p.wpg = pl.wpg;
-  p.cpb = pl.cpb;
-  p.kw = pl.kw;
-  p.xd = pl.xd;
+  gemm_plan(M, N, K, true, false, &pl, 0, false, 1, true, on_16_bytes(x, w));
+  gemm_take_plan(p, pl);
   return gemm_launch(p, true, S(stream));
 }
 
@@ -385,12 +392,8 @@ int dspark_gemm_i8_g128_x8(const void* x, const float* xscale, int32_t M, int32_
   p.xsc = xscale;
   p.xsc_row = K / 16;
   GemmPlan pl;
-  gemm_plan(M, N, K, true, false, &pl, 0, false, 1, true);
-  p.ksplit = pl.ksplit;
-  p.wpg = pl.wpg;
-  p.cpb = pl.cpb;
-  p.kw = pl.kw;
-  p.xd = pl.xd;
+  gemm_plan(M, N, K, true, false, &pl, 0, false, 1, true, !xscale && on_16_bytes(x, w), true);
+  gemm_take_plan(p, pl);
   return gemm_launch(p, true, S(stream));
 }
 
@@ -423,12 +426,8 @@ int dspark_head_argmax_f16(const void* x, int32_t M, int32_t K, const void* w, i
   p.N = N;
   p.K = K;
   GemmPlan pl;
-  gemm_plan(M, N, K, false, false, &pl);
-  p.ksplit = pl.ksplit;
-  p.wpg = pl.wpg;
-  p.cpb = pl.cpb;
-  p.kw = pl.kw;
-  p.xd = pl.xd;
+  gemm_plan(M, N, K, false, false, &pl, 0, false, 1, false, on_16_bytes(x, w));
+  gemm_take_plan(p, pl);
   p.best_part = static_cast<uint64_t*>(workspace);
   p.best = best_keys;
   return gemm_launch(p, false, S(stream));

@@ -277,23 +277,27 @@ struct GemmParams {
   const _Float16* conv_w;   // [N/3][conv_k]
   _Float16* conv_ring;      // [CONV_RING][N/3]
   int conv_k;
+  // Plans over row-major x and w (read by the host alone, so last: the kernels' argument lines stay as they are):
+  int stream;               // > 0: streamed (gemm_stream_kernel), tiles of that many strips
+  int few;                  // few rows (gemm_few_kernel): wpg groups of 8 rows by kw ranges of K
 };
 constexpr int GEMM_FUSE_CONV = 2;
 
 struct GemmPlan {
-  int ksplit = 1, wpg = 1, cpb = 4, kw = 0, xd = 0, bands = 1;
+  int ksplit = 1, wpg = 1, cpb = 4, kw = 0, xd = 0, bands = 1, stream = 0, few = 0;
 };
 // wpg_req > 0 fixes the strips per workgroup (a fused epilogue's group: 3 for GEMM_FUSE_CONV);
 // xop: X comes in operand order (GemmParams::xop); max_bands > 1: the caller adds up to that many output bands
-// (GemmParams::bands).
+// (GemmParams::bands); stream: x and w are row-major on 16-byte boundaries (a few-row or streamed
+// plan may be taken), x8 with int8 x.
 void gemm_plan(int M, int N, int K, bool i8, bool split, GemmPlan* pl, int wpg_req = 0, bool xop = false,
-               int max_bands = 1, bool gs = false);
+               int max_bands = 1, bool gs = false, bool stream = false, bool x8 = false);
 // Split-K workspace: GEMM_COUNTER_BYTES of arrival counters (one u32 per row group, at the same offset for every shape),
 // then the partials. Zero-filled once; every call leaves its counters at zero.
 constexpr int GEMM_COUNTER_SLOTS = 8192;
 constexpr size_t GEMM_COUNTER_BYTES = GEMM_COUNTER_SLOTS * sizeof(uint32_t);
 size_t gemm_ws_bytes(const GemmPlan& pl, int M, int N);
-size_t gemm_ws_bytes(int M, int N, int K, int wpg_req = 0, bool xop = false);  // for the plan of an int8 GEMM
+size_t gemm_ws_bytes(int M, int N, int K, int wpg_req = 0, bool xop = false, bool stream = false);  // an int8 GEMM's
 int gemm_groups(const GemmPlan& pl, int N);                  // row groups (<= GEMM_COUNTER_SLOTS for a split plan)
 uint32_t* gemm_ws_counters(void* ws);
 float* gemm_ws_partials(void* ws);

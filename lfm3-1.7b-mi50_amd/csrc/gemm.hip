@@ -180,32 +180,31 @@ __device__ void gemm_group_epilogue(const GemmParams& p, const f32x4 (&acc)[TB],
   epi_conv(p, tile, RS, grow0, R, 64 * nw, cs);
 }
 
-// Finished sums of one strip (lane (n, g): rows 16 strip + 4 g + i of token 16 tb + n): the strip's row-argmax key
-// per token when the call asks for it, then the epilogue store.
+// Finished sums of one strip and token block (lane (n, g): rows 16 strip + 4 g + i of token 16 tb + n): the strip's
+// row-argmax key per token when the call asks for it, then the epilogue store.
+__device__ __forceinline__ void gemm_block_out(const GemmParams& p, f32x4 acc, int tb, int strip, int lane, f32x4 sc) {
+  const int n = lane & 15, g = lane >> 4, row0 = strip * 16, t = 16 * tb + n;
+  if (p.best_part) {
+    // fold the lane's 4 rows, then the 4 row groups
+    uint64_t b = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint64_t k = argmax_key(acc[i], (uint32_t)(row0 + 4 * g + i));
+      b = k > b ? k : b;
+    }
+    uint64_t o = shfl_xor_u64(b, 16);
+    b = o > b ? o : b;
+    o = shfl_xor_u64(b, 32);
+    b = o > b ? o : b;
+    if (g == 0 && t < p.M) p.best_part[(size_t)t * (p.N / 16) + strip] = b;
+  }
+  gemm_store(p, t, row0, g, acc, sc);
+}
 template <int TB>
 __device__ __forceinline__ void gemm_strip_out(const GemmParams& p, const f32x4 (&acc)[TB], int strip, int lane,
                                                f32x4 sc) {
-  const int n = lane & 15, g = lane >> 4, row0 = strip * 16;
-  if (p.best_part) {
-    // fold the lane's 4 rows, then the 4 row groups
 #pragma unroll
-    for (int tb = 0; tb < TB; ++tb) {
-      const int t = 16 * tb + n;
-      uint64_t b = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint64_t k = argmax_key(acc[tb][i], (uint32_t)(row0 + 4 * g + i));
-        b = k > b ? k : b;
-      }
-      uint64_t o = shfl_xor_u64(b, 16);
-      b = o > b ? o : b;
-      o = shfl_xor_u64(b, 32);
-      b = o > b ? o : b;
-      if (g == 0 && t < p.M) p.best_part[(size_t)t * (p.N / 16) + strip] = b;
-    }
-  }
-#pragma unroll
-  for (int tb = 0; tb < TB; ++tb) gemm_store(p, 16 * tb + n, row0, g, acc[tb], sc);
+  for (int tb = 0; tb < TB; ++tb) gemm_block_out(p, acc[tb], tb, strip, lane, sc);
 }
 
 constexpr int GEMM_CPOL_COHERENT = 16;  // buffer-op cache policy SC1: device-scope coherent store / load
@@ -456,9 +455,15 @@ __global__ __launch_bounds__(512) void gemm_kernel(GemmParams p) {
 // fixes the summation order, so results do not depend on timing.
 // GS (one token block, int8 weights): per-128-column group scales (p.gscale [K/128][N]): the products of a group's two
 // 64-column chunks go to a fresh accumulator that is scaled by the group's scales of the lane's 4 rows and added in group
-// order (the reference applies the scale per group as well, dspark.hip:553-580). Every range and band starts on an
-// even chunk (gemm_launch checks), so a batch's chunk pairs (cb + 2 j, cb + 2 j + 1) are whole groups, the second one
+// order (the reference applies the scale per group as well, dspark.hip:553-580). Every band (gemm_launch checks) and range
+// (gemm_range_chunks) starts on an even chunk, so a batch's chunk pairs (cb + 2 j, cb + 2 j + 1) are whole groups, the second one
 // absent only at the end of a range.
+// Chunks of each of kw ranges of a band (the last ones shorter or empty): whole 128-column groups with group scales.
+__host__ __device__ inline int gemm_range_chunks(int band_chunks, int kw, bool gs) {
+  const int c = (band_chunks + kw - 1) / kw;
+  return gs ? c + (c & 1) : c;
+}
+
 template <int CPW>
 __device__ __forceinline__ void gscale_load(const GemmParams& p, u32x2 (&gsr)[CPW / 2], int cb, int c1, int r4) {
 #pragma unroll
@@ -535,6 +540,14 @@ __device__ __forceinline__ u32x4 x8_transpose4(u32x4 v) {
   return u32x4{c[0], c[1], d[0], d[1]};
 }
 
+// x8_code of two packed values: the product by a mixed-precision fma (x inv - 0, the product rounded once), and one packed
+// conversion of the two integers (exact at any rounding).
+__device__ __forceinline__ uint32_t x8_code_pair(uint32_t xx, float inv) {
+  const half2v h = __builtin_bit_cast(half2v, xx);
+  const float a = rintf(fmaf((float)h[0], inv, -0.f)), b = rintf(fmaf((float)h[1], inv, -0.f));
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+}
+
 // p.x8 == 1: quantize piece g of a chunk, whole in lane (n, g) (lo: its columns 0 .. 7, hi: 8 .. 15); returns its scale
 // and turns lo and hi into codes. max|x| is taken on the fp16 bit patterns.
 __device__ __forceinline__ float x8_quantize_piece(u32x4& lo, u32x4& hi) {
@@ -543,14 +556,11 @@ __device__ __forceinline__ float x8_quantize_piece(u32x4& lo, u32x4& hi) {
   const uint32_t m2 = pmax_u16(pmax_u16(m4[0], m4[1]), pmax_u16(m4[2], m4[3]));
   const float s = x8_piece_scale(x8_mag_value(max(m2 & 0xffffu, m2 >> 16)));
   const float inv = __builtin_amdgcn_rcpf(s);
-  half8 a = as_half8(lo), b = as_half8(hi);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    a[j] = x8_code(a[j], inv);
-    b[j] = x8_code(b[j], inv);
+  for (int j = 0; j < 4; ++j) {
+    lo[j] = x8_code_pair(lo[j], inv);
+    hi[j] = x8_code_pair(hi[j], inv);
   }
-  lo = __builtin_bit_cast(u32x4, a);
-  hi = __builtin_bit_cast(u32x4, b);
   return s;
 }
 // The chunk's 4 pieces in the products' order (xq[p] of lane (n, g): columns 4 g .. 4 g + 3 of piece p) and their scales,
@@ -610,7 +620,7 @@ __device__ __forceinline__ f32x4 x8_scales_load(const GemmParams& p, int n, int 
 // X8: 0 fp16 x; 1 int8 x quantized as it is loaded (p.x8 == 1); 2 int8 codes + scales given (p.x8 == 2).
 // TO (int8 x): tile-major weights; else row-major ones, loaded 16 bytes a lane as everywhere and put in the products'
 // order in registers. (Gathered there as four dword loads each fetched 16 of every 64 bytes: 15360 x 2048 at 8 tokens
-// @A@, 2048 x 7680 @B@.)
+// 32.3 us against 14.8, 2048 x 7680 42.8 against 16.1.)
 template <int TB, bool I8, int CPW, bool XD, int MAXT = 1024, bool GS = false, int X8 = 0, bool ONEB = false,
           bool TO = false>
 __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
@@ -645,7 +655,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
   const int chunks = p.K / 64;
   const int cpb_ = (chunks + p.bands - 1) / p.bands;  // chunks per band
   const int b0 = min(chunks, band * cpb_), b1 = min(chunks, b0 + cpb_);
-  const int cpk = (b1 - b0 + KW - 1) / KW;
+  const int cpk = gemm_range_chunks(b1 - b0, KW, GS);
   const int c0 = min(b1, b0 + kq * cpk), c1 = min(b1, c0 + cpk);
 
   f32x4 acc[TB];
@@ -823,8 +833,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     __builtin_amdgcn_s_barrier();
     if constexpr (X8 == 1) {
       // x quantized where it lies, each chunk once in the workgroup (lane (n, g): token n's piece g): the products below
-      // then read codes and scales as the norm would have left them. (Quantized by each of the strips' waves as they
-      // read it: @C@.)
+      // then read codes and scales as the norm would have left them.
       for (int j = wave_u; j < bc; j += nw) {
         u32x4* xr = xs + (size_t)j * 2 * 64 + lane;
         u32x4 lo = xr[0], hi = xr[64];
@@ -984,6 +993,320 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
   gemm_strip_out<TB>(p, acc, strip, lane, gemm_row_scales_f32(rsc));
 }
 
+// ---------------------------------------------------------------- streamed GEMM over row-major operands
+// Weights [N][K] and x [M][K] as callers keep them, read in whole 128-byte lines: a workgroup owns RS 16-row strips (a
+// tile) and a share of K and streams 128 bytes of every weight row per step (128 int8 or 64 fp16 columns, and the same
+// columns of every token's x) through a ring of SLOTS LDS slots, SLOTS - 1 steps in flight, by direct-to-LDS loads: 8
+// weight rows, or 4 or 8 tokens, per load. In a slot, 16-byte piece q of row r lies in place q ^ (r % 8) of its row, so an
+// operand read (16 rows, one piece each) covers every bank. Wave w multiplies strip w % RS by token blocks w / RS, w / RS
+// + NW / RS, ... Loads past the last row, token or step give zeros or repeat (their products are never stored), so every
+// step issues the same loads and the waits are counted. Tiles beyond one per workgroup follow each other in the same
+// stream (no new fill of the ring). K split over workgroups (p.ksplit): the partials and the last arrival's sum as in
+// gemm_kernel.
+// Bound by HBM (one token block: 5.1 TB/s of weights at 65536 x 2048) and, with more tokens, by the LDS reads of x that each
+// strip's wave makes. Measured against the K-sliced and split kernels on row-major operands: 16384 x 2048 and 2048 x 8192
+// at 16 tokens 12.2 and 11.2 -> 9.7 and 9.6 us, at 64 tokens 21.5 and 21.1 -> 12 and 14; 128000 x 2048 at 16 tokens with its
+// argmax 68.3 -> 58.6, at 64 118 -> 84; fp16 16384 x 2048 at 64 tokens 34.4 -> 19.7.
+// GS (one token block): per-128-column group scales, one group per step: the step's products go to a fresh accumulator
+// that is scaled and added, as in the K-sliced kernel; its rows' scales ride in the slot, one copy per wave.
+constexpr int GEMM_STREAM_WGS = 256;  // one workgroup per CU (the ring)
+template <int TB, int WB, int RS, int NW, int SLOTS, bool GS>
+__global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p) {
+  constexpr int TG = NW / RS, TBW = (TB + TG - 1) / TG;         // token groups; token blocks of a wave
+  constexpr int XB = 256 / WB;                                  // bytes of a token's x per step
+  constexpr int XOFF = RS * 2048, SOFF = XOFF + TB * 16 * XB;   // x and group scales in a slot
+  constexpr int SLOT = SOFF + (GS ? NW * 256 : 0);
+  constexpr int WU = 2 * RS, UNITS = WU + TB * 16 * XB / 1024;  // 1 KB loads of a step, weights first
+  constexpr int LPW = (UNITS + NW - 1) / NW;
+  constexpr int WAIT = (LPW + (GS ? 1 : 0)) * (SLOTS - 2);      // loads younger than the step about to be used
+  static_assert(NW % RS == 0 && WU % NW == 0 && WAIT < 64 && SLOTS >= 3 && SLOTS <= 8, "a counted wait; slots named below");
+  static_assert(!GS || (TB == 1 && WB == 1 && RS <= 8), "group scales: one token block, int8 weights");
+  __shared__ __attribute__((aligned(16))) char slot0[SLOT], slot1[SLOT], slot2[SLOT];
+  __shared__ __attribute__((aligned(16))) char slot3[SLOTS > 3 ? SLOT : 16], slot4[SLOTS > 4 ? SLOT : 16];
+  __shared__ __attribute__((aligned(16))) char slot5[SLOTS > 5 ? SLOT : 16], slot6[SLOTS > 6 ? SLOT : 16];
+  __shared__ __attribute__((aligned(16))) char slot7[SLOTS > 7 ? SLOT : 16], trash[1024];
+  char* const slots[8] = {slot0, slot1, slot2, slot3, slot4, slot5, slot6, slot7};
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = wave % RS, tg = wave / RS;
+  const int strips = p.N / 16, tiles = (strips + RS - 1) / RS;
+  const int ks = blockIdx.x % p.ksplit, tile0 = blockIdx.x / p.ksplit, tstep = gridDim.x / p.ksplit;
+  const int steps = p.K * WB / 128, spk = (steps + p.ksplit - 1) / p.ksplit;
+  const int k0 = ks * spk, nk = min(steps, k0 + spk) - k0;  // (>= 1: the plan's splits are never empty)
+  const int mine = (tiles - tile0 + tstep - 1) / tstep;     // tiles of this workgroup
+  const int total = mine * nk;
+
+  const uint32_t wrow = (uint32_t)p.K * WB, xrow = (uint32_t)p.K * 2;  // bytes of a row
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, (short)0, (int)((uint32_t)p.N * wrow), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, (short)0, (int)((uint32_t)p.M * xrow), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.gscale, (short)0, GS ? (int)((uint32_t)(p.K / 128) * p.N * 2) : 0, 0x00020000);
+  uint32_t off[LPW];  // of step k0 of the first tile
+#pragma unroll
+  for (int i = 0; i < LPW; ++i) {
+    const int u = wave + NW * i;
+    if (i < WU / NW) {
+      off[i] = (uint32_t)(tile0 * 16 * RS + 8 * u + (lane >> 3)) * wrow + (uint32_t)k0 * 128 + (((lane & 7) ^ (lane >> 3)) * 16);
+    } else {
+      constexpr int PT = XB / 16;  // pieces of a token
+      const int t = (64 / PT) * (u - WU) + lane / PT;
+      off[i] = (uint32_t)t * xrow + (uint32_t)k0 * XB + (((lane % PT) ^ (t & 7)) * 16);
+    }
+  }
+  uint32_t goff = 2 * lane < 16 * RS ? ((uint32_t)k0 * p.N + tile0 * 16 * RS + 2 * lane) * 2 : 0x80000000u;
+  // the next step to issue: its place in the share of K, its tile's rows past the first tile's
+  int ik = 0, left = total;
+  uint32_t irow = 0;
+  auto issue = [&](char* slot) {
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) {
+      const int u = wave + NW * i;
+      const bool isw = i < WU / NW, live = LPW * NW == UNITS || u < UNITS;
+      char* dst = live ? slot + u * 1024 : trash;
+      const uint32_t o = !live ? 0x80000000u : off[i] + (isw ? (uint32_t)ik * 128 + irow * wrow : (uint32_t)ik * XB);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(isw ? rw : rx, (__attribute__((address_space(3))) void*)dst, 16, o, 0, 0,
+                                               0);
+    }
+    if constexpr (GS) {
+      const uint32_t o = goff + ((uint32_t)ik * p.N + irow) * 2;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (__attribute__((address_space(3))) void*)(slot + SOFF + wave * 256), 4, o,
+                                               0, 0, 0);
+    }
+    if (--left > 0 && ++ik == nk) {  // (past the last step: the last one again)
+      ik = 0;
+      irow += tstep * 16 * RS;
+    }
+  };
+
+  // Without group scales each of a step's products (per 64 columns, two), and with tiles of 4 strips of every second step,
+  // has an accumulator of its own until the share's end: fewer roundings in a row than the K-sliced kernel's ranges have
+  // (their error passes into the fp16 outputs of the gated epilogue as last-bit flips), and independent products.
+  constexpr int PS = 4 / WB, NC = GS ? 1 : PS * (RS == 4 ? 2 : 1);
+  f32x4 part[TBW][NC], acc[TBW];
+  const f32x4 z4 = {0, 0, 0, 0};
+  auto clear = [&]() {
+#pragma unroll
+    for (int t = 0; t < TBW; ++t)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) part[t][j] = z4;
+  };
+  auto gather = [&]() {
+#pragma unroll
+    for (int t = 0; t < TBW; ++t) {
+#pragma unroll
+      for (int half = NC / 2; half > 0; half /= 2)
+#pragma unroll
+        for (int j = 0; j < half; ++j) part[t][j] += part[t][j + half];
+      acc[t] = part[t][0];
+    }
+  };
+  clear();
+  const int wq = (16 * s + n) * 128, sw = n & 7;
+  int kk = 0, tile = tile0;
+  auto finish = [&]() {  // the tile's products are complete
+    const int strip = tile * RS + s;
+    if (strip >= strips) return;
+    const f32x4 sc = gemm_row_scales_f32(gemm_row_scales(p, strip * 16 + 4 * g));
+#pragma unroll
+    for (int i = 0; i < TBW; ++i)
+      if (tg + TG * i < TB) gemm_block_out(p, acc[i], tg + TG * i, strip, lane, sc);
+  };
+  auto step = [&](int u, const char* cur, char* nxt) {  // u: the step's slot (a constant once unrolled)
+    ring_barrier<WAIT>();  // the step is in LDS; every wave is done with the one before (its slot is nxt)
+    issue(nxt);
+    half4 gs;
+    f32x4 t0 = z4;
+    if constexpr (GS) gs = *reinterpret_cast<const half4*>(cur + SOFF + wave * 256 + (16 * s + 4 * g) * 2);
+#pragma unroll
+    for (int c = 0; c < 2 / WB; ++c) {  // 64 columns each
+      half8 a[2];
+      if constexpr (WB == 1) {
+        const u32x4 w = *reinterpret_cast<const u32x4*>(cur + wq + ((4 * c + g) ^ sw) * 16);
+        a[0] = i8x8_to_half8(w[0], w[1]);
+        a[1] = i8x8_to_half8(w[2], w[3]);
+      } else {
+        a[0] = *reinterpret_cast<const half8*>(cur + wq + ((2 * g) ^ sw) * 16);
+        a[1] = *reinterpret_cast<const half8*>(cur + wq + ((2 * g + 1) ^ sw) * 16);
+      }
+#pragma unroll
+      for (int i = 0; i < TBW; ++i) {
+        const char* xb = cur + XOFF + (16 * min(tg + TG * i, TB - 1) + n) * XB;
+        const half8 b0 = *reinterpret_cast<const half8*>(xb + ((8 * c + 2 * g) ^ sw) * 16);
+        const half8 b1 = *reinterpret_cast<const half8*>(xb + ((8 * c + 2 * g + 1) ^ sw) * 16);
+        f32x4& d0 = GS ? t0 : part[i][GS ? 0 : (PS * u + 2 * c) % NC];
+        f32x4& d1 = GS ? t0 : part[i][GS ? 0 : (PS * u + 2 * c + 1) % NC];
+        d0 = mfma16x16x32(a[0], b0, d0);
+        d1 = mfma16x16x32(a[1], b1, d1);
+      }
+    }
+    if constexpr (GS) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[0][0][r] = fmaf(t0[r], (float)gs[r], part[0][0][r]);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < SLOTS - 1; ++u) issue(slots[u]);
+  // (several tiles: nk is a multiple of SLOTS, so a tile ends where the unrolled steps do)
+  int k = 0;
+  for (; k + SLOTS <= total; k += SLOTS) {
+#pragma unroll
+    for (int u = 0; u < SLOTS; ++u) step(u, slots[u], slots[(u + SLOTS - 1) % SLOTS]);
+    kk += SLOTS;
+    if (kk == nk && p.ksplit == 1) {
+      gather();
+      finish();
+      clear();
+      kk = 0;
+      tile += tstep;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < SLOTS - 1; ++u)
+    if (k + u < total) step(u, slots[u], slots[(u + SLOTS - 1) % SLOTS]);
+  __builtin_amdgcn_s_waitcnt(GEMM_VMCNT0);  // (no load may land once the workgroup's LDS is another's)
+  gather();
+  if (p.ksplit == 1) {
+    if (tile < tiles) finish();  // (one tile, and nk no multiple of SLOTS)
+    return;
+  }
+  // one tile per workgroup: its partials, its arrival, and the last arrival's sum, as in gemm_kernel
+  const int strip = tile * RS + s, row0 = strip * 16;
+  const bool live = strip < strips;
+  const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+      p.part, (short)0, (int)((size_t)p.ksplit * p.M * p.N * sizeof(float)), 0x00020000);
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < TBW; ++i) {
+      const int t = 16 * (tg + TG * i) + n;
+      if (t < p.M)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i]), rp,
+                                               (uint32_t)((((size_t)ks * p.M + t) * p.N + row0 + 4 * g) * sizeof(float)), 0,
+                                               GEMM_CPOL_COHERENT);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(GEMM_VMCNT0);
+  __syncthreads();
+  __shared__ int last_s;
+  if (threadIdx.x == 0) {
+    const uint32_t old = __hip_atomic_fetch_add(p.counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last_s = old == (uint32_t)(p.ksplit - 1);
+    if (last_s) __hip_atomic_store(p.counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!last_s || !live) return;
+#pragma unroll
+  for (int i = 0; i < TBW; ++i) {
+    const int t = min(16 * (tg + TG * i) + n, p.M - 1);
+    u32x4 v[GEMM_FIXUP_BATCH];
+    f32x4 sum = z4;
+    for (int q0 = 0; q0 < p.ksplit; q0 += GEMM_FIXUP_BATCH) {
+#pragma unroll
+      for (int q = 0; q < GEMM_FIXUP_BATCH; ++q)
+        v[q] = __builtin_amdgcn_raw_buffer_load_b128(
+            rp, (uint32_t)((((size_t)min(q0 + q, p.ksplit - 1) * p.M + t) * p.N + row0 + 4 * g) * sizeof(float)), 0,
+            GEMM_CPOL_COHERENT);
+#pragma unroll
+      for (int q = 0; q < GEMM_FIXUP_BATCH; ++q)
+        if (q0 + q < p.ksplit) sum += __builtin_bit_cast(f32x4, v[q]);
+    }
+    acc[i] = sum;
+  }
+  finish();
+}
+
+// ---------------------------------------------------------------- few rows over row-major operands
+// For up to 16 tokens and so few rows that 16-row strips leave CUs idle or need K split over workgroups: a workgroup owns
+// S groups of 8 rows and all of K, its waves the S groups by KW ranges of K. An operand's 16 rows are 8 weight rows twice:
+// lane (n, g) holds row n % 8, columns 64 (n / 8) + 16 g .. of a pair of chunks (so a load is 8 whole 128-byte lines), x
+// likewise token n % 8. Of a product's four 8 x 8 quadrants the two on the diagonal are then the chunks' own products
+// (rows by tokens); they are added at the end, the others never read. One token block of 8 costs what 16 tokens cost
+// a 16-row strip per chunk pair, from twice the workgroups. The ranges' sums meet in LDS in range order: no workspace, no
+// second pass.
+// Group scales (a pair is a group); X8: int8 x, each piece quantized by the lane that holds it (the K-sliced kernel's
+// x8_quantize). (Row scales have a workspace and split K over workgroups of the streamed kernel: x crosses into each CU
+// once per split there, whole here, which at 16 tokens is 4 times the weights: 2048 x 8192 9.5 against 12.8 us.)
+// Measured, 2048 x 7680: fp16 x 8 tokens 8.0 us, 16 tokens 12.9; int8 x 8 tokens 10.3 (42.8 with 128
+// workgroups of one strip and 7 ranges).
+// PB: pairs per batch, every load of which is issued before its first product (the loads of x are the kernel's bound, so a
+// range shorter than four pairs takes a shorter batch rather than repeat its last pair).
+template <int TB, bool X8, int PB>
+__global__ __launch_bounds__(1024) void gemm_few_kernel(GemmParams p) {
+  extern __shared__ u32x4 xs[];
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int S = p.wpg, KW = p.kw, s = wave % S, kq = wave / S;
+  const int groups = p.N / 8;
+  const int grp = min((int)blockIdx.x * S + s, groups - 1);
+  const int row0 = grp * 8;
+  // the thread's output quad
+  const int e = threadIdx.x, oq = e % 16, otb = e / 16 % TB, os = e / (16 * TB);
+  const int orow = (blockIdx.x * S + os) * 8 + 4 * (oq >> 3), ot = 8 * otb + (oq & 7);
+  const bool out = os < S && orow < p.N;
+  const int pairs = p.K / 128, ppw = (pairs + KW - 1) / KW;
+  const int p0 = min(pairs, kq * ppw), p1 = min(pairs, p0 + ppw);
+  const uint8_t* wl = reinterpret_cast<const uint8_t*>(p.w) + (size_t)(row0 + (n & 7)) * p.K + 64 * (n >> 3) + 16 * g;
+  const _Float16* xl[TB];
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb)  // (tokens past M feed only outputs that are never stored)
+    xl[tb] = p.x + (size_t)min(8 * tb + (n & 7), p.M - 1) * p.K + 64 * (n >> 3) + 16 * g;
+  const _Float16* gl = p.gscale + row0 + 4 * (g & 1);
+  f32x4 acc[TB];
+  const f32x4 z4 = {0, 0, 0, 0};
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb) acc[tb] = z4;
+  for (int pb = p0; pb < p1; pb += PB) {
+    u32x4 w[PB], xb[PB][TB][2];
+    u32x2 gsr[PB];
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int c = min(pb + i, p1 - 1);
+      w[i] = ldg_nt(reinterpret_cast<const u32x4*>(wl + (size_t)c * 128));
+      gsr[i] = ldg(reinterpret_cast<const u32x2*>(gl + (size_t)c * p.N));
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) {
+        xb[i][tb][0] = ldg(reinterpret_cast<const u32x4*>(xl[tb] + (size_t)c * 128));
+        xb[i][tb][1] = ldg(reinterpret_cast<const u32x4*>(xl[tb] + (size_t)c * 128 + 8));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      if (pb + i >= p1) break;
+      const u32x4 wi = X8 ? x8_transpose4(w[i]) : w[i];
+      const half8 a[2] = {i8x8_to_half8(wi[0], wi[1]), i8x8_to_half8(wi[2], wi[3])};
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) {
+        f32x4 t = z4;
+        if constexpr (X8) {
+          u32x2 xq[4];
+          const f32x4 xs4 = x8_quantize(xb[i][tb][0], xb[i][tb][1], xq);
+          x8_chunk(t, a, xq, xs4);
+        } else {
+          t = mfma16x16x32(a[0], as_half8(xb[i][tb][0]), t);
+          t = mfma16x16x32(a[1], as_half8(xb[i][tb][1]), t);
+        }
+        const half4 gs = __builtin_bit_cast(half4, gsr[i]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[tb][r] = fmaf(t[r], (float)gs[r], acc[tb][r]);
+      }
+    }
+  }
+  // the second chunk's quadrant (tokens n - 8, rows of lane groups 2, 3) onto the first's
+  f32x4* red = reinterpret_cast<f32x4*>(xs);  // [kq][s][tb][16 quads]
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb) {
+    f32x4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = __shfl(acc[tb][r], (lane + 40) & 63);
+    if (n < 8 && g < 2) red[((kq * S + s) * TB + tb) * 16 + 8 * g + n] = acc[tb] + o;
+  }
+  __syncthreads();
+  if (!out) return;
+  f32x4 v = z4;
+  for (int k = 0; k < KW; ++k) v += red[((k * S + os) * TB + otb) * 16 + oq];
+  gemm_store(p, ot, orow, 0, v, f32x4{1, 1, 1, 1});
+}
+
 // Split-K reduce in index order + epilogue: one thread per 4 rows of one token, partial loads in flight in batches.
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p) {
   if (gemm_stopped(p)) return;
@@ -1117,7 +1440,7 @@ static void launch_sliced_tb(const GemmParams& p, hipStream_t s) {
   const int groups = (p.N / 16 + p.wpg - 1) / p.wpg;
   const dim3 grid(groups * p.bands), block(64 * p.wpg * p.kw);
   const size_t lds = gemm_sliced_lds_bytes(p, I8);
-  const int cpk = ((p.K / 64 + p.bands - 1) / p.bands + p.kw - 1) / p.kw;  // chunks per range (of the band's)
+  const int cpk = gemm_range_chunks((p.K / 64 + p.bands - 1) / p.bands, p.kw, p.gscale);  // chunks per range
   if constexpr (I8 && TB == 1) {
     if (p.gscale) {  // group scales: X per wave, or X^T of the band in LDS at once (gemm_launch checked)
       if (p.x8 == 1) {  // int8 x (LFM3_X8), quantized as it is loaded
@@ -1173,8 +1496,62 @@ static void launch_sliced_tb(const GemmParams& p, hipStream_t s) {
   hipLaunchKernelGGL((gemm_sliced_kernel<TB, I8, 8, false>), grid, block, lds, s, p);
 }
 
+// Streamed plans: p.stream strips a tile; rings of 8 slots while they fit LDS, else 4 (divisors of the steps of K = 2048).
+template <int TB, int WB, int RS, int NW, int SLOTS, bool GS>
+static void launch_stream_as(const GemmParams& p, hipStream_t s) {
+  const int tiles = (p.N / 16 + RS - 1) / RS, steps = p.K * WB / 128;
+  const bool follow = p.ksplit == 1 && steps % SLOTS == 0;  // tiles one after the other in a workgroup's stream
+  const dim3 grid(follow ? std::min(tiles, GEMM_STREAM_WGS) : tiles * p.ksplit), block(64 * NW);
+  hipLaunchKernelGGL((gemm_stream_kernel<TB, WB, RS, NW, SLOTS, GS>), grid, block, 0, s, p);
+}
+template <int TB, int WB, bool GS>
+static void launch_stream_tb(const GemmParams& p, hipStream_t s) {
+  if constexpr (!GS) {
+    if (p.stream == 8) {
+      launch_stream_as<TB, WB, 8, 8, 4, false>(p, s);
+      return;
+    }
+  }
+  launch_stream_as<TB, WB, 4, TB == 1 ? 4 : 8, TB <= 2 ? 8 : 4, GS>(p, s);
+}
+template <bool I8>
+static void launch_stream(const GemmParams& p, hipStream_t s) {
+  constexpr int WB = I8 ? 1 : 2;
+  if constexpr (I8) {
+    if (p.gscale) {
+      launch_stream_tb<1, 1, true>(p, s);
+      return;
+    }
+  }
+  switch ((p.M + 15) / 16) {
+    case 1: launch_stream_tb<1, WB, false>(p, s); break;
+    case 2: launch_stream_tb<2, WB, false>(p, s); break;
+    case 3: launch_stream_tb<3, WB, false>(p, s); break;
+    default: launch_stream_tb<4, WB, false>(p, s); break;
+  }
+}
+
+template <int TB, bool X8>
+static void launch_few_as(const GemmParams& p, hipStream_t s) {
+  const dim3 grid((p.N / 8 + p.wpg - 1) / p.wpg), block(64 * p.wpg * p.kw);
+  const size_t lds = (size_t)p.wpg * p.kw * TB * 256;
+  const int ppw = (p.K / 128 + p.kw - 1) / p.kw;  // pairs per range
+  auto kernel = ppw == 1 ? gemm_few_kernel<TB, X8, 1> : ppw == 2 ? gemm_few_kernel<TB, X8, 2> : gemm_few_kernel<TB, X8, 4>;
+  hipLaunchKernelGGL(kernel, grid, block, lds, s, p);
+}
+static void launch_few(const GemmParams& p, hipStream_t s) {
+  if (p.M > 8)
+    p.x8 ? launch_few_as<2, true>(p, s) : launch_few_as<2, false>(p, s);
+  else
+    p.x8 ? launch_few_as<1, true>(p, s) : launch_few_as<1, false>(p, s);
+}
+
 template <bool I8>
 static void launch_gemm(const GemmParams& p, hipStream_t s) {
+  if (p.stream) {
+    launch_stream<I8>(p, s);
+    return;
+  }
   const int tb = (p.M + 15) / 16;
   if (p.kw > 0) {
     switch (tb) {
@@ -1279,11 +1656,10 @@ static bool gemm_plan_sliced(int N, int K, int tb, bool i8, int wpg_req, bool xo
       KW = std::min(8, std::max(4, (gbc + 7) / 8));
       xd = true;
     }
-    while (KW > 1 && ((gbc + KW - 1) / KW) % 2) --KW;
   }
   // X^T through LDS: all token blocks at once when they fit 64 KB, else one token block per pass, each pass's X^T
   // within 64 KB and each range within one 8-chunk batch (its weights stay in registers)
-  const int bc = (chunks + bands - 1) / bands, cpk = (bc + KW - 1) / std::max(1, KW);
+  const int bc = (chunks + bands - 1) / bands, cpk = gemm_range_chunks(bc, std::max(1, KW), gs);
   const int tp = gemm_pass_tbs(tb, bc);
   if (!xd && ((size_t)tp * bc * 2048 > GEMM_X_LDS || (tp < tb && cpk > 8) || (tb > 2 && cpk > 8))) return false;
   pl->ksplit = 1;
@@ -1295,8 +1671,44 @@ static bool gemm_plan_sliced(int N, int K, int tb, bool i8, int wpg_req, bool xo
   return true;
 }
 
-void gemm_plan(int M, int N, int K, bool i8, bool split, GemmPlan* pl, int wpg_req, bool xop, int max_bands, bool gs) {
+// Few-row plans (row-major operands on 16-byte boundaries): one group of 8 rows per workgroup while those are at most one
+// per CU, else two.
+static bool gemm_plan_few(int M, int N, int K, bool gs, GemmPlan* pl) {
+  if (!gs || M > 16 || K % 128 || N > 16 * GEMM_STREAM_WGS) return false;
+  *pl = GemmPlan{};
+  pl->few = 1;
+  pl->wpg = N > 8 * GEMM_STREAM_WGS ? 2 : 1;
+  pl->kw = std::min(16 / pl->wpg, K / 128);
+  return true;
+}
+
+// Streamed plans (row-major operands on 16-byte boundaries, whole 128-byte steps; others take the plans below). Tiles of 4
+// strips, or of 8 for int8 weights where the busiest CU then has no more strips (half the x traffic: 128000 x 2048 at 64
+// tokens 84 against 91 us, but 40000 rows 40.4 against 39.0; fp16 weights, whose x is half as much, 154 against 147 us at
+// 128000 rows). K over workgroups until every CU has one, at least 4 steps each. Group scales have no workspace and so no
+// split: below 128 tiles they stay with the K-sliced plans.
+static bool gemm_plan_stream(int M, int N, int K, bool i8, bool split, bool gs, GemmPlan* pl) {
+  const int wb = i8 ? 1 : 2, strips = N / 16, steps = K * wb / 128;
+  if ((size_t)K * wb % 128 || (size_t)N * K * wb >= (size_t)1 << 31 || (size_t)M * K * 2 >= (size_t)1 << 31) return false;
+  if (gs && M > 16) return false;
+  const auto per_cu = [&](int rs) { return rs * ((strips + rs * GEMM_STREAM_WGS - 1) / (rs * GEMM_STREAM_WGS)); };
+  const int rs = i8 && !gs && per_cu(8) <= per_cu(4) ? 8 : 4;
+  const int tiles = (strips + rs - 1) / rs;
+  if (gs && tiles < GEMM_STREAM_WGS / 2) return false;  // (no workspace, no split)
+  int ks = 1;
+  while (split && tiles * ks * 2 <= GEMM_STREAM_WGS && steps / (2 * ks) >= 4) ks *= 2;
+  const int spk = (steps + ks - 1) / ks;
+  *pl = GemmPlan{};
+  pl->stream = pl->wpg = rs;
+  pl->ksplit = (steps + spk - 1) / spk;  // (no empty share)
+  return true;
+}
+
+void gemm_plan(int M, int N, int K, bool i8, bool split, GemmPlan* pl, int wpg_req, bool xop, int max_bands, bool gs,
+               bool stream, bool x8) {
   const int strips = N / 16, chunks = K / 64, tb = (M + 15) / 16;
+  if (stream && gemm_plan_few(M, N, K, gs, pl)) return;
+  if (stream && !x8 && gemm_plan_stream(M, N, K, i8, split, gs, pl)) return;
   if (gemm_plan_sliced(N, K, tb, i8, wpg_req, xop, max_bands, pl, gs)) return;
   pl->kw = 0;
   pl->bands = 1;
@@ -1319,9 +1731,9 @@ size_t gemm_ws_bytes(const GemmPlan& pl, int M, int N) {
   return GEMM_COUNTER_BYTES + (((size_t)pl.ksplit * M * N * sizeof(float) + 255) / 256) * 256;
 }
 
-size_t gemm_ws_bytes(int M, int N, int K, int wpg_req, bool xop) {
+size_t gemm_ws_bytes(int M, int N, int K, int wpg_req, bool xop, bool stream) {
   GemmPlan pl;
-  gemm_plan(M, N, K, true, true, &pl, wpg_req, xop);
+  gemm_plan(M, N, K, true, true, &pl, wpg_req, xop, 1, false, stream);
   return gemm_ws_bytes(pl, M, N);
 }
 
@@ -1336,6 +1748,16 @@ float* gemm_ws_partials(void* ws) { return reinterpret_cast<float*>(static_cast<
 #endif
 
 int gemm_launch(GemmParams& p, bool i8, hipStream_t s) {
+  if (p.few) {
+    if (!i8 || p.xop || p.yop || p.tiled || p.fuse || p.x8 > 1 || p.ysc || p.bands > 1 || p.st || p.best_part || p.M > 16 ||
+        p.K % 128 || !p.gscale || p.scale || p.ksplit != 1 || p.wpg * p.kw > 16)
+      return DSPARK_EINVAL;
+    launch_few(p, s);
+    return (int)hipGetLastError();
+  }
+  if (p.stream && (p.xop || p.yop || p.tiled || p.fuse || p.x8 || p.ysc || p.bands > 1 || p.st || p.M > 64 ||
+                   (p.gscale && (!i8 || p.M > 16 || p.scale || p.ksplit != 1)) || (p.ksplit > 1 && !p.counters)))
+    return DSPARK_EINVAL;
   if ((p.xop && p.xop < (p.M + 15) / 16) || (p.yop && p.yop < (p.M + 15) / 16)) return DSPARK_EINVAL;
   // group scales: the K-sliced kernel, one token block, whole 128-column groups in every band and range, X per wave or
   // the band's X^T in LDS at once, no row scales
@@ -1348,10 +1770,10 @@ int gemm_launch(GemmParams& p, bool i8, hipStream_t s) {
     const bool conv = p.fuse == GEMM_FUSE_CONV && p.wpg == 3 && p.y16;
     if (!p.gscale || (!gated && !conv) || p.ysc_row < (gated ? p.N / 32 : p.N / 48)) return DSPARK_EINVAL;
   }
-  if (p.gscale) {
+  if (p.gscale && !p.stream) {
     if (!i8 || p.kw <= 0 || p.M > 16 || p.K % 128 || p.scale) return DSPARK_EINVAL;
-    const int bands = std::max(1, p.bands), bc = (p.K / 64 + bands - 1) / bands, cpk = (bc + p.kw - 1) / p.kw;
-    if ((bands > 1 && bc % 2) || cpk % 2 || (!gemm_sliced_xd(p, i8) && (size_t)bc * 2048 > GEMM_X_LDS) ||
+    const int bands = std::max(1, p.bands), bc = (p.K / 64 + bands - 1) / bands;
+    if ((bands > 1 && bc % 2) || (!gemm_sliced_xd(p, i8) && (size_t)bc * 2048 > GEMM_X_LDS) ||
         (gemm_sliced_xd(p, i8) && p.wpg * p.kw > 8))
       return DSPARK_EINVAL;
   }
@@ -1365,7 +1787,7 @@ int gemm_launch(GemmParams& p, bool i8, hipStream_t s) {
         gemm_sliced_lds_bytes(p, i8) > GEMM_X_LDS + (p.x8 == 1 ? gemm_x8_scale_bytes(bc) : 0))
       return DSPARK_EINVAL;
     // X^T in passes (it does not fit LDS for every token block at once): each range within one batch of weights
-    const int cpk = (bc + p.kw - 1) / p.kw;
+    const int cpk = gemm_range_chunks(bc, p.kw, p.gscale);
     const int tp = gemm_pass_tbs(tb, bc);
     if (!gemm_sliced_xd(p, i8) && ((size_t)tp * bc * 2048 > GEMM_X_LDS || (tp < tb && cpk > 8) || (tb > 2 && cpk > 8)))
       return DSPARK_EINVAL;
@@ -1373,7 +1795,7 @@ int gemm_launch(GemmParams& p, bool i8, hipStream_t s) {
     if (p.bands > 1 && (p.epilogue != 0 || !p.y32 || p.y16 || p.best_part || p.fuse || p.bands > p.K / 64))
       return DSPARK_EINVAL;
   }
-  if (!DSPARK_GEMM_FIXUP) p.counters = nullptr;
+  if (!DSPARK_GEMM_FIXUP && !p.stream) p.counters = nullptr;
   if (p.fuse && p.ksplit > 1 && !p.counters) return DSPARK_EINVAL;  // a fused epilogue needs the in-kernel fixup
   if (i8)
     launch_gemm<true>(p, s);
