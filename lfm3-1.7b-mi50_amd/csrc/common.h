@@ -71,15 +71,38 @@ __device__ __forceinline__ void ring_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Butterfly over a whole wave without the LDS unit (a shuffle there costs about 100 cycles a level): level by level each
+// lane's value is combined with lane ^ 32's and lane ^ 16's by the half-wave swaps, then with lane ^ 8's, ^ 4's, ^ 2's
+// and ^ 1's by row rotations -- after a level the values repeat with half the period, so that a rotation by 4 in a row of
+// 16 brings lane ^ 4's value, and so on. The same pairs in the same order as an xor-shuffle butterfly, hence the same bits
+// (the operations commute). Every lane of the wave must be active.
+template <int N>
+__device__ __forceinline__ uint32_t row_ror(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x120 + N, 0xf, 0xf, false);
+}
+template <typename F>
+__device__ __forceinline__ uint32_t wave_butterfly(uint32_t v, F op) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  v = op(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = op(b[0], b[1]);
+  v = op(v, row_ror<8>(v));
+  v = op(v, row_ror<4>(v));
+  v = op(v, row_ror<2>(v));
+  return op(v, row_ror<1>(v));
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
+  return __uint_as_float(wave_butterfly(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+    return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b)));
+  }));
 }
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  return __uint_as_float(wave_butterfly(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+    return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
+  }));
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  return wave_butterfly(v, [](uint32_t a, uint32_t b) { return max(a, b); });
 }
 
 // quantize_pair (kernels/ops.hip:212-224) of a record's 128 values, one IEEE fp32 operation per step: the scale from
@@ -93,10 +116,12 @@ __device__ __forceinline__ int rec_code(float x, float inv) {
 
 // Argmax key (reference dspark.hip:967-971): ordered float bits above, 0xFFFFFFFF - index below. The maximum key is the
 // largest value and, among equal values, the smallest index.
-__device__ __forceinline__ uint64_t argmax_key(float v, uint32_t idx) {
+__device__ __forceinline__ uint32_t argmax_ord(float v) {  // float bits in the order of the values
   const uint32_t u = __float_as_uint(v);
-  const uint32_t ord = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-  return ((uint64_t)ord << 32) | (uint64_t)(0xffffffffu - idx);
+  return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+}
+__device__ __forceinline__ uint64_t argmax_key(float v, uint32_t idx) {
+  return ((uint64_t)argmax_ord(v) << 32) | (uint64_t)(0xffffffffu - idx);
 }
 
 // K/V page formats (one block of PAGE keys x D dims per (page, KV head)). K is stored in the operand order of
@@ -123,13 +148,11 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
   return ((uint64_t)hi << 32) | lo;
 }
 
+// (every lane of the wave active) The largest high word, then the largest low word under it.
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint64_t w = shfl_xor_u64(v, o);
-    v = w > v ? w : v;
-  }
-  return v;
+  const uint32_t hi = wave_max_u32((uint32_t)(v >> 32));
+  const uint32_t lo = wave_max_u32((uint32_t)(v >> 32) == hi ? (uint32_t)v : 0u);
+  return ((uint64_t)hi << 32) | lo;
 }
 
 }  // namespace dspark

@@ -495,49 +495,51 @@ __global__ __launch_bounds__(256) void markov_table_kernel(const int8_t* w1q, co
 // j - 1's key, so its dots are row ci of the table and its values fmaf(T[ci][r], w2s[r] * s1c[ci], base[j][r]) are
 // markov_kernel's bit for bit; the confidence test and the writes of tokens, M and the per-step keys are
 // markov_kernel's and markov_finalize's. Step 0 (previous token = the anchor, any vocabulary id) stays with
-// markov_kernel. Thread t owns rows 16 t .. 16 t + 15 (N <= 16384), so a step is one table row read with all its
-// loads in flight, then a workgroup argmax.
-constexpr int CHAIN_THREADS = 1024, CHAIN_ROWS = 16, CHAIN_MAX_N = CHAIN_THREADS * CHAIN_ROWS;
+// markov_kernel. Thread t owns rows 4 t .. 4 t + 3 of each 4096 (N <= 16384), so a step is one table row read with all its
+// loads in flight, each a contiguous kilobyte of the wave, then a workgroup argmax (the keys carry their row: the order of
+// the rows over the threads does not matter). Bound by the table row's latency and one CU's load rate: 14 steps of 16384
+// rows 34.1 us (44.7 with the argmax of 64-bit keys by LDS shuffles; 53.4 with that and 16 rows in a row per thread, whose
+// loads touched 64 lines each).
+constexpr int CHAIN_THREADS = 1024, CHAIN_QUADS = 4, CHAIN_STRIDE = 4 * CHAIN_THREADS;
+constexpr int CHAIN_MAX_N = CHAIN_QUADS * CHAIN_STRIDE;
 __global__ __launch_bounds__(1024) void markov_chain_kernel(MarkovParams p) {
   __shared__ uint64_t red[2][CHAIN_THREADS / 64];  // double-buffered by step parity: one barrier per step
   dspark_state* st = p.st;
   if (stopped(st)) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int N = p.N, r0 = CHAIN_ROWS * tid;
-  const bool live = r0 < N;  // N % 16 == 0: a thread's rows are all inside or all outside
-  f32x4 s2[CHAIN_ROWS / 4];
+  const int N = p.N, r0 = 4 * tid;  // rows r0 + CHAIN_STRIDE i .. + 3
+  const auto live = [&](int i) { return r0 + CHAIN_STRIDE * i < N; };  // (N % 16 == 0: four rows are all inside or outside)
+  f32x4 s2[CHAIN_QUADS];
 #pragma unroll
-  for (int i = 0; i < CHAIN_ROWS / 4; ++i)
-    s2[i] = live ? ldg(reinterpret_cast<const f32x4*>(p.w2s + r0) + i) : f32x4{0, 0, 0, 0};
+  for (int i = 0; i < CHAIN_QUADS; ++i)
+    s2[i] = live(i) ? ldg(reinterpret_cast<const f32x4*>(p.w2s + r0 + CHAIN_STRIDE * i)) : f32x4{0, 0, 0, 0};
   const int cap = draft_cap(st, p.max_drafts, p.max_drafts_dev, p.block);
   int M = st->M;  // nonzero when step 0's confidence test stopped drafting
   uint64_t key = 0;
   if (M == 0 && cap >= 1) key = __hip_atomic_load(p.best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // A step's base row and confidence word do not depend on the previous step's argmax: each is loaded one step ahead
   // (with the current step's table row), so only the table row's latency lies on the chain.
-  f32x4 bv[CHAIN_ROWS / 4];
+  f32x4 bv[CHAIN_QUADS];
   float bconf = 0.f;
-  auto base_row = [&](int j, f32x4 (&b)[CHAIN_ROWS / 4], float& c) {
+  auto base_row = [&](int j, f32x4 (&b)[CHAIN_QUADS], float& c) {
     const float* brow = p.base + (size_t)j * p.stride;
-    if (live) {
 #pragma unroll
-      for (int i = 0; i < CHAIN_ROWS / 4; ++i) b[i] = ldg(reinterpret_cast<const f32x4*>(brow + r0) + i);
-    }
+    for (int i = 0; i < CHAIN_QUADS; ++i)
+      if (live(i)) b[i] = ldg(reinterpret_cast<const f32x4*>(brow + r0 + CHAIN_STRIDE * i));
     c = ldg(brow + N);
   };
   if (M == 0 && cap >= 2) base_row(1, bv, bconf);
   for (int j = 1; j < cap && M == 0; ++j) {
     const uint32_t ci = 0xffffffffu - (uint32_t)key;
-    f32x4 tv[CHAIN_ROWS / 4];
-    if (live) {
-      const f32x4* trow = reinterpret_cast<const f32x4*>(p.table + (size_t)ci * N + r0);
+    f32x4 tv[CHAIN_QUADS];
+    const float* trow = p.table + (size_t)ci * N + r0;
 #pragma unroll
-      for (int i = 0; i < CHAIN_ROWS / 4; ++i) tv[i] = ldg(trow + i);
-    }
+    for (int i = 0; i < CHAIN_QUADS; ++i)
+      if (live(i)) tv[i] = ldg(reinterpret_cast<const f32x4*>(trow + CHAIN_STRIDE * i));
     const int prev = ldg(p.crop_ids + ci);
     const float s1 = ldg(p.s1c + ci);
     const float conf = bconf + ldg(p.c2c + ci) + p.conf_bias;
-    f32x4 bn[CHAIN_ROWS / 4];
+    f32x4 bn[CHAIN_QUADS];
     float bnconf = 0.f;
     base_row(min(j + 1, cap - 1), bn, bnconf);  // the last step reloads its own row (unused)
     if (!(conf >= p.conf_thr)) {
@@ -549,26 +551,26 @@ __global__ __launch_bounds__(1024) void markov_chain_kernel(MarkovParams p) {
       break;
     }
     if (tid == 0) st->tokens[j] = prev;
-    uint64_t best = 0;
-    if (live) {
+    // the thread's largest value and its first row (rows in rising order: a later one has to be larger)
+    uint32_t bo = 0, br = 0xffffffffu;
 #pragma unroll
-      for (int i = 0; i < CHAIN_ROWS / 4; ++i)
+    for (int i = 0; i < CHAIN_QUADS; ++i)
+      if (live(i)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const uint64_t k = argmax_key(fmaf(tv[i][e], s2[i][e] * s1, bv[i][e]), (uint32_t)(r0 + 4 * i + e));
-          best = k > best ? k : best;
+          const uint32_t o = argmax_ord(fmaf(tv[i][e], s2[i][e] * s1, bv[i][e]));
+          br = o > bo ? (uint32_t)(r0 + CHAIN_STRIDE * i + e) : br;
+          bo = max(o, bo);
         }
-    }
-    best = wave_max_u64(best);
+      }
+    const uint64_t best = wave_max_u64(((uint64_t)bo << 32) | (0xffffffffu - br));
     // red[j & 1] was last read in step j - 2, before every thread passed step j - 1's barrier
     if (lane == 0) red[j & 1][wave] = best;
     __syncthreads();
-    key = red[j & 1][0];
-#pragma unroll
-    for (int w = 1; w < CHAIN_THREADS / 64; ++w) key = red[j & 1][w] > key ? red[j & 1][w] : key;
+    key = wave_max_u64(red[j & 1][lane & (CHAIN_THREADS / 64 - 1)]);
     if (tid == 0) p.best[j] = key;
 #pragma unroll
-    for (int i = 0; i < CHAIN_ROWS / 4; ++i) bv[i] = bn[i];
+    for (int i = 0; i < CHAIN_QUADS; ++i) bv[i] = bn[i];
     bconf = bnconf;
   }
   if (p.plant) {
