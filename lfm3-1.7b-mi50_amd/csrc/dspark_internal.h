@@ -238,46 +238,55 @@ __device__ __forceinline__ float x8_mag_value(uint32_t bits) {
 __device__ __forceinline__ _Float16 x8_code(_Float16 x, float inv) { return (_Float16)rintf((float)x * inv); }
 
 struct GemmParams {
+  // The first two 64-byte lines hold what the K-sliced kernel needs before its first loads, so that they come in one round
+  // trip.
   const struct ::dspark_state* st;  // when set, a stopped round (run == 0) skips the launch's work
   const _Float16* x;        // [M][K]
   const void* w;            // [N][K] biased int8 or fp16
   const _Float16* scale;    // [N] or nullptr
   const _Float16* gscale;   // or [K / 128][N]: one fp16 scale per (128-column group, row), the reference's per-128
                             // format (internal/weights/quant.go:66-104); K-sliced plans with one token block only
-  float* y32;               // [M][N]
-  _Float16* y16;            // [M][N] ([M][N/2] for the gated epilogue)
-  float* part;              // split-K partials [ksplit][M][N]
-  uint64_t* best_part;      // row-argmax keys per strip [M][N/16] (head) or nullptr
-  uint64_t* best;           // [M]
-  int M, N, K, ksplit, epilogue;
-  uint32_t* counters;       // split-K arrival counter per group (zero between calls); nullptr: separate reduce kernel
-  int wpg;                  // waves (16-row strips) per workgroup (gemm_plan)
-  int cpb;                  // 64-column chunks per weight-load batch: 4 or 8 (gemm_plan)
-  int kw;                   // > 0: K-sliced plan, workgroups of wpg strips x kw ranges of K (ksplit 1, gemm_plan)
-  int xd;                   // K-sliced, int8, one token block: each wave loads its own range of X (no LDS staging)
-  int bands;                // K-sliced, > 1: K in `bands` shares over as many workgroups, band b's scaled sums to
-                            // y32 + b M N (epilogue 0, y32 only): the caller adds the bands (the norm kernel does)
+  const float* xsc;         // x8 == 2
+  int M, N, K;
   int xop;                  // > 0: x in operand order (xop_elem) with xop >= ceil(M / 16) token blocks; 0: row-major
-  int yop;                  // > 0: the fp16 output y16 in operand order with yop token blocks (for the next GEMM's X)
+
+  int wpg;                  // waves (16-row strips) per workgroup (gemm_plan)
+  int kw;                   // > 0: K-sliced plan, workgroups of wpg strips x kw ranges of K (ksplit 1, gemm_plan)
+  int wpg_inv;              // K-sliced: ceil(65536 / wpg), wave / wpg = wave wpg_inv >> 16 (gemm_launch sets these three)
+  int band_chunks;          // K-sliced: chunks per band
+  int range_chunks;         // K-sliced: chunks per range (gemm_range_chunks)
   int tiled;                // int8 weights tile-major: [N / 16][K / 64][1 KB tile], lane l's 16 B at 16 l
   // Fused row-group epilogue (the group's scaled products go through LDS; y32 is not written):
   //   GEMM_FUSE_CONV: each group is 16 channels [B, C, X] of the conv mix (48 rows): gated short conv, y16 [M][N/3]
   //     and the conv history ring at st->a + t (conv_wave)
   int fuse;
+  int xsc_row;
+  int bands;                // K-sliced, > 1: K in `bands` shares over as many workgroups, band b's scaled sums to
+                            // y32 + b M N (epilogue 0, y32 only): the caller adds the bands (the norm kernel does)
+  int conv_k;
+  const _Float16* conv_w;   // [N/3][conv_k]
+  _Float16* conv_ring;      // [CONV_RING][N/3]
+  int epilogue;
+  int yop;                  // > 0: the fp16 output y16 in operand order with yop token blocks (for the next GEMM's X)
+
+  float* y32;               // [M][N]
+  _Float16* y16;            // [M][N] ([M][N/2] for the gated epilogue)
+  uint64_t* best_part;      // row-argmax keys per strip [M][N/16] (head) or nullptr
+  uint64_t* best;           // [M]
   // LFM3_X8 (with gscale only): 1 x is fp16, quantized per 16-column piece as it is loaded; 2 x holds int8 codes as
   // integer-valued halves and xsc their fp32 scales, [token][xsc_row] with piece k / 16 of token t at t xsc_row + k / 16
   int x8;
-  const float* xsc;
-  int xsc_row;
   // LFM3_X8 output (gated epilogue 1 of a K-sliced plan with an even number of strips per workgroup and one band, or
   // GEMM_FUSE_CONV; group scales only): y16 receives the int8 codes of the fp16 outputs and ysc their scales,
   // [token][ysc_row] with output column c's piece at t ysc_row + c / 16 (the next GEMM reads them with x8 = 2)
-  float* ysc;
   int ysc_row;
-  const _Float16* conv_w;   // [N/3][conv_k]
-  _Float16* conv_ring;      // [CONV_RING][N/3]
-  int conv_k;
-  // Plans over row-major x and w (read by the host alone, so last: the kernels' argument lines stay as they are):
+  float* ysc;
+  float* part;              // split-K partials [ksplit][M][N]
+  uint32_t* counters;       // split-K arrival counter per group (zero between calls); nullptr: separate reduce kernel
+  int ksplit;
+  int cpb;                  // 64-column chunks per weight-load batch: 4 or 8 (gemm_plan)
+  int xd;                   // K-sliced, int8, one token block: each wave loads its own range of X (no LDS staging)
+  // Plans over row-major x and w:
   int stream;               // > 0: streamed (gemm_stream_kernel), tiles of that many strips
   int few;                  // few rows (gemm_few_kernel): wpg groups of 8 rows by kw ranges of K
 };

@@ -207,6 +207,7 @@ __device__ __forceinline__ void gemm_strip_out(const GemmParams& p, const f32x4 
   for (int tb = 0; tb < TB; ++tb) gemm_block_out(p, acc[tb], tb, strip, lane, sc);
 }
 
+constexpr int GEMM_CPOL_NT = 2;         // buffer-op cache policy NT: each weight byte has one reader
 constexpr int GEMM_CPOL_COHERENT = 16;  // buffer-op cache policy SC1: device-scope coherent store / load
 // s_waitcnt immediate: vmcnt(n) (6 bits, split low 4 / high 2), other counters left unconstrained
 #define GEMM_VMCNT(n) ((((n) & 15) | (((n) >> 4) << 14)) | 0x0F70)
@@ -459,17 +460,19 @@ __global__ __launch_bounds__(512) void gemm_kernel(GemmParams p) {
 // (gemm_range_chunks) starts on an even chunk, so a batch's chunk pairs (cb + 2 j, cb + 2 j + 1) are whole groups, the second one
 // absent only at the end of a range.
 // Chunks of each of kw ranges of a band (the last ones shorter or empty): whole 128-column groups with group scales.
-__host__ __device__ inline int gemm_range_chunks(int band_chunks, int kw, bool gs) {
+inline int gemm_range_chunks(int band_chunks, int kw, bool gs) {
   const int c = (band_chunks + kw - 1) / kw;
   return gs ? c + (c & 1) : c;
 }
 
+// (rg: the buffer p.gscale; voff: the lane's 4 rows)
 template <int CPW>
-__device__ __forceinline__ void gscale_load(const GemmParams& p, u32x2 (&gsr)[CPW / 2], int cb, int c1, int r4) {
+__device__ __forceinline__ void gscale_load(const GemmParams& p, __amdgpu_buffer_rsrc_t rg, u32x2 (&gsr)[CPW / 2], int cb,
+                                            int c1, uint32_t voff) {
 #pragma unroll
   for (int j = 0; j < CPW / 2; ++j) {
     const int c = min(cb + 2 * j, c1 - 1);
-    gsr[j] = ldg(reinterpret_cast<const u32x2*>(p.gscale + (size_t)(c >> 1) * p.N + r4));
+    gsr[j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rg, voff, (c >> 1) * p.N * 2, 0));
   }
 }
 
@@ -500,19 +503,6 @@ __device__ __forceinline__ void gscale_products(f32x4& acc, const u32x2 (&gsr)[C
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4 mfma16x16x16(half4v a, half4v b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-}
-
-// Token n's 4 halves of piece p of chunk c (lane (g, n)): operand-order x at p.x (xop), or row-major.
-struct X8Src {
-  const _Float16* base;  // this lane's first 4 halves of chunk 0, piece 0
-  size_t cstride, pstride;
-};
-__device__ __forceinline__ X8Src x8_src(const GemmParams& p, int g, int n) {
-  if (p.xop) {
-    // xop_elem(n, 64 c + 16 p + 4 g + j) = (((c tbs) 2 + g / 2) 64 + 16 p + n) 8 + 4 (g % 2) + j
-    return X8Src{p.x + ((size_t)(g >> 1) * 64 + n) * 8 + 4 * (g & 1), (size_t)p.xop * 1024, 128};
-  }
-  return X8Src{p.x + (size_t)min(n, p.M - 1) * p.K + 4 * g, 64, 16};
 }
 
 // Per-half max of two packed pairs of fp16 magnitudes: for non-negative halves the order of the bit patterns as
@@ -612,11 +602,6 @@ __device__ __forceinline__ void gemm_gated_x8_out(const GemmParams& p, f32x4 v, 
   if ((strip & 1) == 0 && g == 0) p.ysc[(size_t)t * p.ysc_row + strip / 2] = sc;
 }
 
-// Token n's 4 piece scales of chunk c (p.x8 == 2).
-__device__ __forceinline__ f32x4 x8_scales_load(const GemmParams& p, int n, int c) {
-  return ldg(reinterpret_cast<const f32x4*>(p.xsc + (size_t)min(n, p.M - 1) * p.xsc_row + 4 * c));
-}
-
 // X8: 0 fp16 x; 1 int8 x quantized as it is loaded (p.x8 == 1); 2 int8 codes + scales given (p.x8 == 2).
 // TO (int8 x): tile-major weights; else row-major ones, loaded 16 bytes a lane as everywhere and put in the products'
 // order in registers. (Gathered there as four dword loads each fetched 16 of every 64 bytes: 15360 x 2048 at 8 tokens
@@ -629,15 +614,19 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
   static_assert(!ONEB || (XD && MAXT > 512), "the one-batch form is the 1024-thread X-per-wave kernel's");
   // The stop flag is loaded first and tested once the data loads are in flight and the products computed (before
   // anything is stored), so its latency overlaps theirs; a stopped round writes nothing.
+  // The prologue up to the first weight load is on every launch's critical path (a round is a chain of some two hundred
+  // launches, half of them this kernel): no integer division, the arguments' first lines in one round trip, and buffer loads
+  // whose chunk offset is one scalar. (With divisions by the plan's numbers and 64-bit addresses per chunk it was 420
+  // instructions, about 0.8 us a launch: 16-layer rounds 1087 -> 1057 us, reference geometry 1389 -> 1372.)
+  asm volatile("" ::"s"(p.st), "s"(p.wpg), "s"(p.conv_ring));
   const int run = run_flag_load(p.st);
   extern __shared__ u32x4 xs[];
   constexpr int WV = I8 ? 1 : 2;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int n = lane & 15, g = lane >> 4;
   const int S = p.wpg, KW = p.kw;
-  const int s = wave % S, kq = wave / S;
-  const int groups = (p.N / 16 + S - 1) / S;
-  const int grp = blockIdx.x % groups, band = blockIdx.x / groups;  // band: a share of K (bands > 1)
+  const int kq = wave * p.wpg_inv >> 16, s = wave - kq * S;
+  const int grp = blockIdx.x, band = blockIdx.y;  // band: a share of K (bands > 1)
   const int strips = p.N / 16;
   const int strip_raw = grp * S + s;
   const bool live = strip_raw < strips;
@@ -653,32 +642,32 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     conv_stage_issue(p, grp * 16, wave, nw, lane, conv_ring_lds, conv_w_lds);
   }
   const int chunks = p.K / 64;
-  const int cpb_ = (chunks + p.bands - 1) / p.bands;  // chunks per band
+  const int cpb_ = p.band_chunks;
   const int b0 = min(chunks, band * cpb_), b1 = min(chunks, b0 + cpb_);
-  const int cpk = gemm_range_chunks(b1 - b0, KW, GS);
-  const int c0 = min(b1, b0 + kq * cpk), c1 = min(b1, c0 + cpk);
+  const int c0 = min(b1, b0 + kq * p.range_chunks), c1 = min(b1, c0 + p.range_chunks);
 
   f32x4 acc[TB];
 #pragma unroll
   for (int tb = 0; tb < TB; ++tb) acc[tb] = f32x4{0, 0, 0, 0};
 
   const bool tiled = X8 ? TO : I8 && p.tiled;
-  const uint8_t* wrow = tiled ? reinterpret_cast<const uint8_t*>(p.w) + (size_t)strip * chunks * 1024 + lane * 16
-                              : reinterpret_cast<const uint8_t*>(p.w) + (size_t)(row0 + n) * p.K * (I8 ? 1 : 2) + 16 * g;
-  const int cstride = tiled ? 1024 : 64;
+  // the strip's weights (16 rows of K: the same bytes in either layout), lane and chunk strides within them
+  const int wbytes = p.K * (I8 ? 1 : 2);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(reinterpret_cast<const uint8_t*>(p.w) + (size_t)strip * 16 * wbytes), (short)0, 16 * wbytes, 0x00020000);
+  const uint32_t wvo = tiled ? (uint32_t)lane * 16 : (uint32_t)n * wbytes + (I8 ? 16 : 32) * g;
+  const int cstride = tiled ? 1024 : 64 * (I8 ? 1 : 2);
+  const __amdgpu_buffer_rsrc_t rgs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.gscale, (short)0, GS ? (p.K >> 7) * p.N * 2 : 0, 0x00020000);
+  const uint32_t gvo = (uint32_t)(row0 + 4 * g) * 2;
   // chunk cb + i, clamped to the last valid chunk (a re-read of a line just fetched, discarded): the number of loads
   // issued is CPW * WV on every path, so the counted wait for X below stays exact
   auto load = [&](u32x4 (&w)[CPW][WV], int cb) {
 #pragma unroll
     for (int i = 0; i < CPW; ++i) {
-      const int c = min(cb + i, max(c1, 1) - 1);
-      if (I8) {
-        w[i][0] = ldg_nt(reinterpret_cast<const u32x4*>(wrow + (size_t)c * cstride));
-      } else {
-        const u32x4* wp = reinterpret_cast<const u32x4*>(wrow + 2 * c * 64 + 16 * g);
-        w[i][0] = ldg_nt(wp);
-        w[i][WV - 1] = ldg_nt(wp + 1);
-      }
+      const int so = min(cb + i, max(c1, 1) - 1) * cstride;
+      w[i][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wvo, so, GEMM_CPOL_NT));
+      if (!I8) w[i][WV - 1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wvo + 16, so, GEMM_CPOL_NT));
     }
   };
   auto weights = [&](const u32x4 (&wr)[WV], half8 (&a)[2]) {
@@ -697,8 +686,18 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     // lane (n, g): token n (min(n, M - 1) row-major: rows past M feed only output columns that are never stored),
     // 16 B at columns 64 c + 16 g and 64 c + 16 g + 8 of chunk c; in operand order those are lane l's 16 B of the two
     // 1 KB blocks of chunk c
-    const _Float16* xb0 = p.xop ? p.x + lane * 8 : p.x + (size_t)min(n, p.M - 1) * p.K + 16 * g;
-    const size_t xcs = p.xop ? (size_t)p.xop * 1024 : 64, xhs = p.xop ? 512 : 8;  // halves per chunk, per half
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)p.x, (short)0, (p.xop ? 16 * p.xop : p.M) * p.K * 2, 0x00020000);
+    const int xcs = p.xop ? p.xop * 2048 : 128, xhs = p.xop ? 1024 : 16;  // bytes per chunk, per half
+    const uint32_t xvo = p.xop ? (uint32_t)lane * 16 : (uint32_t)(min(n, p.M - 1) * p.K + 16 * g) * 2;
+    // int8 codes (X8 == 2): 4 halves of piece pc, at lane (n, g)'s columns 4 g of it; xop_elem(n, 64 c + 16 pc + 4 g + j) =
+    // (((c tbs) 2 + g / 2) 64 + 16 pc + n) 8 + 4 (g % 2) + j
+    const int xps = p.xop ? 256 : 32;  // bytes per piece
+    const uint32_t x8vo =
+        p.xop ? (uint32_t)((g >> 1) * 64 + n) * 16 + 8 * (g & 1) : (uint32_t)(min(n, p.M - 1) * p.K + 4 * g) * 2;
+    const __amdgpu_buffer_rsrc_t rxs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)p.xsc, (short)0, X8 == 2 ? p.M * p.xsc_row * 4 : 0, 0x00020000);
+    const uint32_t xsvo = (uint32_t)(min(n, p.M - 1) * p.xsc_row) * 4;
     // One batch: its X and weight loads, then its products. The first batch is outside the loop: at a loop head the
     // compiler's wait for the previous iteration's loads would also hold the first batch back behind the flag load.
     // Token block tb of chunk c (operand order, TB > 1 needs it): the next 1 KB block pair, tb * 1024 halves on.
@@ -710,21 +709,22 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
 #pragma unroll
       for (int i = 0; i < CPW; ++i) {
         const int c = min(cb + i, c1 - 1);
+        const int so = c * xcs;
         if constexpr (X8 == 2) {
-          const X8Src xsrc = x8_src(p, g, n);
 #pragma unroll
           for (int pc = 0; pc < 4; ++pc)
-            xq[i][pc] = ldg(reinterpret_cast<const u32x2*>(xsrc.base + (size_t)c * xsrc.cstride + pc * xsrc.pstride));
-          xsl[i] = x8_scales_load(p, n, c);
+            xq[i][pc] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rx, x8vo + pc * xps, so, 0));
+          xsl[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rxs, xsvo, c * 16, 0));
         } else {
 #pragma unroll
           for (int tb = 0; tb < TB; ++tb) {
-            xb[i][tb][0] = ldg(reinterpret_cast<const u32x4*>(xb0 + (size_t)c * xcs + tb * 1024));
-            xb[i][tb][1] = ldg(reinterpret_cast<const u32x4*>(xb0 + (size_t)c * xcs + tb * 1024 + xhs));
+            xb[i][tb][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xvo + tb * 2048, so, 0));
+            xb[i][tb][1] =
+                __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xvo + tb * 2048 + xhs, so, 0));
           }
         }
       }
-      if constexpr (GS) gscale_load<CPW>(p, gsr, cb, c1, row0 + 4 * g);
+      if constexpr (GS) gscale_load<CPW>(p, rgs, gsr, cb, c1, gvo);
       load(w, cb);
       // every load of the batch issued before its first product (the scheduler would otherwise reuse a consumed
       // chunk's registers for the last loads, a round trip after the first products)
@@ -796,14 +796,16 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     const int tbp = gemm_pass_tbs(TB, cpb_);  // token blocks per stage (the host sizes LDS the same way)
     const bool all = tbp >= TB;
     auto stage = [&](int t0, int nt) {
-      for (int r = wave_u; r < nt * bc * 2; r += nw) {
-        const int h = r & 1, j = b0 + (r >> 1) % bc, tb = t0 + (r >> 1) / bc;
-        const int t = 16 * tb + n;
+      for (int u = 0; u < nt; ++u) {
+        const int tb = t0 + u, t = 16 * tb + n;
         if (t < p.M) {
-          const uint32_t off = p.xop ? (uint32_t)(((((size_t)j * p.xop + tb) * 2 + h) * 64 + lane) * 16)
-                                     : (uint32_t)(((size_t)t * p.K + j * 64 + 16 * g + 8 * h) * 2);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(xs + r * 64), 16, off,
-                                                   0, 0, 0);
+          const uint32_t vo = p.xop ? (uint32_t)(tb * 2048 + lane * 16) : (uint32_t)(t * p.K + 16 * g) * 2;
+          for (int r = wave_u; r < bc * 2; r += nw) {
+            const uint32_t off = vo + (p.xop ? (uint32_t)(b0 + (r >> 1)) * (p.xop * 2048) + (r & 1) * 1024
+                                             : (uint32_t)(b0 + (r >> 1)) * 128 + (r & 1) * 16);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rx, (__attribute__((address_space(3))) void*)(xs + (u * bc * 2 + r) * 64), 16, off, 0, 0, 0);
+          }
         }
       }
     };
@@ -826,7 +828,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
         }
       }
     }
-    if constexpr (GS) gscale_load<CPW>(p, gsr, c0, c1, row0 + 4 * g);  // older than X: covered by the wait below
+    if constexpr (GS) gscale_load<CPW>(p, rgs, gsr, c0, c1, gvo);  // older than X: covered by the wait below
     stage(0, min(tbp, TB));
     load(w, c0);
     __builtin_amdgcn_s_waitcnt(GEMM_VMCNT(CPW * WV));
@@ -847,7 +849,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     if constexpr (X8) {  // one token block, X^T of the band in LDS at once, as below
       for (int cb = c0; cb < c1; cb += CPW) {
         if (cb != c0) {
-          gscale_load<CPW>(p, gsr, cb, c1, row0 + 4 * g);
+          gscale_load<CPW>(p, rgs, gsr, cb, c1, gvo);
           load(w, cb);
         }
         f32x4 accg = f32x4{0, 0, 0, 0};
@@ -878,7 +880,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     } else if constexpr (GS) {  // one token block, X^T of the band in LDS at once (gemm_launch checked)
       for (int cb = c0; cb < c1; cb += CPW) {
         if (cb != c0) {
-          gscale_load<CPW>(p, gsr, cb, c1, row0 + 4 * g);
+          gscale_load<CPW>(p, rgs, gsr, cb, c1, gvo);
           load(w, cb);
         }
         gscale_products<CPW>(acc[0], gsr, cb, c1, [&](int i, f32x4 t) {
@@ -1438,9 +1440,9 @@ static void launch_sliced_x8(const GemmParams& p, dim3 grid, dim3 block, size_t 
 template <int TB, bool I8>
 static void launch_sliced_tb(const GemmParams& p, hipStream_t s) {
   const int groups = (p.N / 16 + p.wpg - 1) / p.wpg;
-  const dim3 grid(groups * p.bands), block(64 * p.wpg * p.kw);
+  const dim3 grid(groups, p.bands), block(64 * p.wpg * p.kw);
   const size_t lds = gemm_sliced_lds_bytes(p, I8);
-  const int cpk = gemm_range_chunks((p.K / 64 + p.bands - 1) / p.bands, p.kw, p.gscale);  // chunks per range
+  const int cpk = p.range_chunks;
   if constexpr (I8 && TB == 1) {
     if (p.gscale) {  // group scales: X per wave, or X^T of the band in LDS at once (gemm_launch checked)
       if (p.x8 == 1) {  // int8 x (LFM3_X8), quantized as it is loaded
@@ -1788,6 +1790,9 @@ int gemm_launch(GemmParams& p, bool i8, hipStream_t s) {
       return DSPARK_EINVAL;
     // X^T in passes (it does not fit LDS for every token block at once): each range within one batch of weights
     const int cpk = gemm_range_chunks(bc, p.kw, p.gscale);
+    p.wpg_inv = (65536 + p.wpg - 1) / p.wpg;
+    p.band_chunks = bc;
+    p.range_chunks = cpk;
     const int tp = gemm_pass_tbs(tb, bc);
     if (!gemm_sliced_xd(p, i8) && ((size_t)tp * bc * 2048 > GEMM_X_LDS || (tp < tb && cpk > 8) || (tb > 2 && cpk > 8)))
       return DSPARK_EINVAL;
