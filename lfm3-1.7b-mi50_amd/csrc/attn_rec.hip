@@ -15,16 +15,22 @@
 // The output is the softmax of those scores over the dequantized V, the reference's fp64 claim (accuracy against an
 // fp64 attention of the same int8 Q/K/V, benchmarks/verify_attention.txt).
 //
-// gfx950 mapping. A workgroup owns one key split of every KV head (the records of a position's heads are
-// interleaved, so a page is one contiguous 33 KB read): wave (h, rg) holds QB 16-row blocks of KV head h. Pages
-// stream through a 3-slot LDS ring with direct-to-LDS loads; per page the workgroup first expands V into a
-// transposed fp16 copy (V^T chunks in the operand order of the PV product) and gathers the page's scales, then each
-// wave runs
+// gfx950 mapping. A workgroup owns one key split of one KV head: wave rg holds QB 16-row blocks. Its pages (the head's
+// 32 records of 264 bytes, 1056 apart) stream through a 3-slot LDS ring with direct-to-LDS loads; per page the workgroup
+// first expands V into a transposed fp16 copy (V^T chunks in the operand order of the PV product) and gathers the
+// page's scales, then each wave runs
 //   S^T[keys][rows] = K8[keys][128] * Q8^T      on v_mfma_i32_16x16x32_i8, one product per 32-dim group (exact)
 //   O^T[128][rows] += V^T[128][keys] * P^T      on v_mfma_f32_16x16x32_f16
 // with the lazy running max of the fp16 kernels (a row's max moves only when a score passes it by more than TAU, so
 // p <= 2^TAU); P is scaled by PSCALE 2^-TAU, which keeps P below the reference's bound (v scale x 4096) and rounds
 // it at the same relative point. Splits write the fp16 kernels' partial format; attn_combine_kernel merges them.
+//
+// What bounds it: a workgroup's chain per page (wait, expand, barrier, products: ~1.1 us alone on its CU) and ~5 us before
+// and after its pages, so the work is split by head as well as by key range: four heads' workgroups in 40 KB of LDS each
+// share a CU and fill each other's waits, and the same number of workgroups leaves a quarter of the partials to merge.
+// Against one workgroup per split for all four heads (whole 33 KB pages, one workgroup a CU), six layers with their
+// merges: 8 tokens at 256 / 4096 / 32771 / 131072 keys 69.7 / 91.5 / 144.2 / 259.8 -> 53.2 / 70.9 / 128.4 / 246.5 us, 16
+// tokens 91.4 / 123.6 / 197.8 / 354.8 -> 57.0 / 80.2 / 158.4 / 340.4.
 #include "common.h"
 #include "dspark.h"
 #include "dspark_internal.h"
@@ -37,14 +43,20 @@ typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 constexpr int REC_D = 128;
 constexpr int REC_BYTES = 2 * REC_D + 8;                 // 264
 constexpr int REC_KVH = 4;                               // KV heads the attention kernel takes (the reference's)
-constexpr int REC_PAGE = PAGE * REC_KVH * REC_BYTES;     // 33792 bytes: 33 chunks of 1 KB
-constexpr int REC_CHUNKS = REC_PAGE / 1024;
+constexpr int REC_PAGE = PAGE * REC_KVH * REC_BYTES;     // 33792 bytes
+// One head's records of a page in LDS: 17 pieces of 16 bytes a record, pieces 0 to 7 the K codes, pieces 8 on from 8
+// bytes earlier in the record (its 264 bytes are no whole number of pieces; no load reads past the record).
+constexpr int LREC = 272, LREC_KS = 136, LREC_V = 140, LREC_VS = 268;
+constexpr int REC_LOADS = (PAGE * 17 + 63) / 64;         // wave loads per page: 9
+constexpr int REC_SLOT = REC_LOADS * 1024;
+constexpr uint32_t REC_NO_PAGE = 65535;                  // no page of a pool under 2 GiB: its loads are out of range
 constexpr int REC_BT_MAX = 1024;                         // pages per split
 constexpr float REC_TAU = 8.f;
 constexpr float REC_PSCALE = 4096.f / 256.f;             // 4096 x 2^-TAU
 constexpr float REC_M_INIT = -1e30f;
 constexpr float REC_QK_SCALE = 0.08838834764831845f * 1.4426950408889634f;  // 1/sqrt(128) x log2(e), in fp32
-static_assert(REC_PAGE % 1024 == 0, "a record page is whole 1 KB chunks");
+
+static_assert((uint64_t)REC_NO_PAGE * REC_PAGE >= 0x80000000ull, "REC_NO_PAGE lies past any pool");
 
 #define DSPARK_LDSP(x) ((__attribute__((address_space(3))) void*)(x))
 
@@ -124,14 +136,12 @@ __device__ __forceinline__ int vt_slot(int l) { return (l + (l >> 3)) * 16; }
 template <int NT>
 __device__ __forceinline__ void rec_expand(const char* page, char* vt, float* kvs) {
   const half2v bias = {(_Float16)1152.f, (_Float16)1152.f};
-  for (int task = threadIdx.x; task < REC_KVH * 4 * 32; task += NT) {
+  for (int task = threadIdx.x; task < 4 * 32; task += NT) {
     const int dq = (task & 3) | (((task >> 3) & 7) << 2), g = ((task >> 2) & 1) | (((task >> 6) & 1) << 1);
-    const int hh = task >> 7;
-    constexpr int KS = REC_KVH * REC_BYTES;  // one position on
-    const char* r0 = page + ((8 * g) * REC_KVH + hh) * REC_BYTES + REC_D + 4 + 4 * dq;
+    const char* r0 = page + 8 * g * LREC + LREC_V + 4 * dq;
     uint32_t w[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) w[k] = *reinterpret_cast<const uint32_t*>(r0 + k * KS) ^ 0x80808080u;
+    for (int k = 0; k < 8; ++k) w[k] = *reinterpret_cast<const uint32_t*>(r0 + k * LREC) ^ 0x80808080u;
     // dims j of keys 0-3 and 4-7: byte j of each key's word
     uint32_t lo[4], hi[4];
 #pragma unroll
@@ -145,7 +155,7 @@ __device__ __forceinline__ void rec_expand(const char* page, char* vt, float* kv
       d[2] = __builtin_amdgcn_perm(y23, y01, 0x05040100u);
       d[3] = __builtin_amdgcn_perm(y23, y01, 0x07060302u);
     }
-    char* base = vt + (hh * 8 + (dq >> 2)) * VT_CHUNK;
+    char* base = vt + (dq >> 2) * VT_CHUNK;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const half2v a = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, lo[j], 0x04010400u)) - bias;
@@ -158,34 +168,36 @@ __device__ __forceinline__ void rec_expand(const char* page, char* vt, float* kv
                 __builtin_bit_cast(uint32_t, e)};
     }
   }
-  for (int e = threadIdx.x; e < REC_KVH * PAGE; e += NT) {
-    const int hh = e / PAGE, key = e % PAGE;
-    const char* rec = page + (key * REC_KVH + hh) * REC_BYTES;
-    kvs[(hh * 2) * PAGE + key] = *reinterpret_cast<const float*>(rec + REC_D);
+  if (threadIdx.x < PAGE) {
+    const int key = threadIdx.x;
+    const char* rec = page + key * LREC;
+    kvs[key] = *reinterpret_cast<const float*>(rec + LREC_KS);
     // v scale x PSCALE (a power of two: fp16(p * (vs * PSCALE)) = fp16(fp32(p * vs) * PSCALE) exactly)
-    kvs[(hh * 2 + 1) * PAGE + key] = *reinterpret_cast<const float*>(rec + 2 * REC_D + 4) * REC_PSCALE;
+    kvs[PAGE + key] = *reinterpret_cast<const float*>(rec + LREC_VS) * REC_PSCALE;
   }
 }
 
-// QB row blocks per wave, NRG row groups per KV head: waves = 4 x NRG, wave w = head w / NRG, row group w % NRG
-// (instantiated with QB = 1).
+// QB row blocks per wave, NRG row groups (waves; instantiated with QB = 1). With 3 waves or more the registers are held to
+// what keeps three workgroups on a CU (208 -> 142 for NRG = 3: 9 tokens at 32771 keys 149 -> 138 us for six layers).
 template <int QB, int NRG>
-__global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(AttnParams p) {
-  constexpr int NW = REC_KVH * NRG, NT = NW * 64;
-  constexpr int LPW = (REC_CHUNKS + NW - 1) / NW;  // page chunk loads per wave
-  __shared__ __attribute__((aligned(16))) char ring0[REC_PAGE], ring1[REC_PAGE], ring2[REC_PAGE];
-  __shared__ __attribute__((aligned(16))) char vt[REC_KVH * 8 * VT_CHUNK];
-  __shared__ __attribute__((aligned(16))) float kvs[REC_KVH * 2 * PAGE];
+__global__ __launch_bounds__(NRG * 64, NRG <= 2 ? 2 : 3) void verify_attn_rec_kernel(AttnParams p) {
+  constexpr int NW = NRG, NT = NW * 64;
+  constexpr int LPW = (REC_LOADS + NW - 1) / NW;  // page loads per wave
+  __shared__ __attribute__((aligned(16))) char ring0[REC_SLOT], ring1[REC_SLOT], ring2[REC_SLOT];
+  __shared__ __attribute__((aligned(16))) char vt[8 * VT_CHUNK];
+  __shared__ __attribute__((aligned(16))) float kvs[2 * PAGE];
   __shared__ __attribute__((aligned(16))) char trash[1024];
-  __shared__ int32_t sm_bt[REC_BT_MAX];
+  __shared__ uint16_t sm_bt[REC_BT_MAX];  // physical pages (a pool under 2 GiB has fewer than REC_NO_PAGE)
   // Every line of the kernel arguments the prologue reads in the first round trip (the split bounds' line, 0xc0 on,
   // would otherwise be read after the State's, one more dependent miss before the block-table loads).
   asm volatile("" ::"s"(p.mix));
   if (p.st && !attn_state_range(p)) return;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = wave / NRG, rg = wave % NRG;
-  const int split = blockIdx.x;
+  const int rg = wave;
+  // workgroups 8 apart share an XCD: the four heads of a split there read the lines their records share from one L2
+  const int h = (int)(blockIdx.x >> 3) & (REC_KVH - 1), split = (int)(blockIdx.x >> 5) * 8 + (int)(blockIdx.x & 7);
+  if (split >= p.S) return;
   const int R = p.nrb * 16;
   const int pb = __builtin_amdgcn_readfirstlane(p.page0 + split * p.pps);
   const int pe = __builtin_amdgcn_readfirstlane(min(pb + p.pps, p.page0 + p.npages));
@@ -193,10 +205,14 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
   p.full_lo = __builtin_amdgcn_readfirstlane(p.full_lo);
   p.full_hi = __builtin_amdgcn_readfirstlane(p.full_hi);
   const bool paged = p.bt != nullptr;
-  if (paged) {
-    for (int i = threadIdx.x; i < nsteps; i += NT) sm_bt[i] = ldg(p.bt + pb + i);
-    __syncthreads();
-  }
+  // The first two pages' table entries by scalar loads, so that their loads wait for nothing else; all of them to LDS
+  // behind those loads, for the steps.
+  int first[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) first[i] = paged && nsteps > 0 ? (int)min((uint32_t)p.bt[pb + min(i, nsteps - 1)], REC_NO_PAGE) : pb + i;
+  const int my_bt = paged && nsteps > 0 ? ldg(p.bt + pb + min((int)threadIdx.x, nsteps - 1)) : 0;
+  if (paged)
+    for (int i = (int)threadIdx.x + NT; i < nsteps; i += NT) sm_bt[i] = (uint16_t)min((uint32_t)ldg(p.bt + pb + i), REC_NO_PAGE);
 
   // Q of the wave's row blocks (padding rows past G*M read the last row; the store skips them)
   constexpr bool FRESH_OK = QB == 1 && NRG <= 3;  // (the host sends a fresh block to these shapes only: 16 waves spill)
@@ -215,32 +231,35 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
   __builtin_amdgcn_sched_barrier(0);  // the Q loads stay ahead of the page loads, so waiting for Q drains no page
 
   const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)p.kp, (short)0, (int)p.k_bytes, 0x00020000);
-  // Page k of the split into `slot`: chunk c < 33 of the page goes to wave c % NW; every wave issues exactly LPW loads
-  // (chunks past the page become out-of-range loads into `trash`), so the counted waits are compile-time constants.
-  auto issue = [&](int k, char* slot) {
-    const int phys = paged ? __builtin_amdgcn_readfirstlane(sm_bt[k]) : pb + k;
+  // Head h's records of page k of the split (physical page `phys`) into `slot`: load c < 9 goes to wave c % NW; every
+  // wave issues exactly LPW loads (loads past the page go to `trash`, pages past the split are out-of-range loads: zeros,
+  // no memory traffic), so the waits are counted.
+  uint32_t loff[LPW];
+#pragma unroll
+  for (int i = 0; i < LPW; ++i) {
+    const uint32_t e = (uint32_t)(wave + i * NW) * 64u + (uint32_t)lane, key = e / 17u, piece = e - 17u * key;
+    loff[i] = key < PAGE ? (key * REC_KVH + (uint32_t)h) * REC_BYTES + 16u * piece - (piece >= 8 ? 8u : 0u) : 0x80000000u;
+  }
+  auto issue = [&](int k, int phys, char* slot) {
     const uint32_t base = (uint32_t)phys * (uint32_t)REC_PAGE;
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
       const int c = wave + i * NW;
-      char* dst = trash;
-      uint32_t off = 0x80000000u;
-      if (c < REC_CHUNKS) {
-        off = base + (uint32_t)c * 1024u + (uint32_t)lane * 16u;
-        dst = slot + c * 1024;
-      }
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, DSPARK_LDSP(dst), 16, off, 0, 0, 2);
+      char* dst = c < REC_LOADS ? slot + c * 1024 : trash;
+      const uint32_t off = k < nsteps && loff[i] < 0x80000000u ? base + loff[i] : 0x80000000u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, DSPARK_LDSP(dst), 16, off, 0, 0, 0);
     }
   };
-  if (nsteps > 0) issue(0, ring0);
-  if (nsteps > 1) issue(1, ring1);
+  issue(0, first[0], ring0);
+  issue(1, first[1], ring1);
+  if (paged && (int)threadIdx.x < nsteps) sm_bt[threadIdx.x] = (uint16_t)min((uint32_t)my_bt, REC_NO_PAGE);
 
   // Fresh block (p.mix): Q and the block's K/V records (positions a .. a + M - 1) from the attention-mix GEMM's rows,
   // the q/k norm + RoPE (+ quantize_pair for the records) done here as the q/k norm + RoPE kernel does. Loaded after
   // the first two pages are in flight (waiting for these loads waits for those pages too, which step 0 needs anyway,
-  // and keeps the raw rows out of registers while the pages are issued). Fresh pair i = (token i / 4, head i % 4) of
-  // this split's pages goes to wave i % NW; the records sit in registers until their page is in LDS.
-  constexpr int FPW = 4;  // fresh pairs per wave at most: 4 M pairs over 4 NRG waves, M <= 4 NRG (the host checks)
+  // and keeps the raw rows out of registers while the pages are issued). The record of token i, if on
+  // this split's pages, goes to wave i % NW; the records sit in registers until their page is in LDS.
+  constexpr int FPW = 4;  // fresh records per wave at most: M over NRG waves, M <= 4 NRG (the host checks)
   uint32_t fkq[FPW], fvq[FPW];  // lanes 0..31: the record's codes of dims l + 32 e, one byte per e
   float fks[FPW], fvs[FPW];
   int fslot[FPW], fpg[FPW];     // position's slot and page (-1: no pair)
@@ -306,7 +325,7 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
     for (int f = 0; f < FPW; ++f) {
       fpg[f] = -1;
       const int i = wave + NW * f;
-      const int t = i / REC_KVH, hh = i % REC_KVH;
+      const int t = i;
       const int pos = p.a + t;
       if (t >= p.M || pos / PAGE < pb || pos / PAGE >= pe) continue;  // wave-uniform
       const float* row = p.mix + (size_t)t * p.mix_row;
@@ -314,8 +333,8 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int d = (lane & 31) + 32 * e;
-        k[e] = row[(size_t)(p.QH + hh) * REC_D + d];
-        v[e] = row[(size_t)(p.QH + p.KVH + hh) * REC_D + d];
+        k[e] = row[(size_t)(p.QH + h) * REC_D + d];
+        v[e] = row[(size_t)(p.QH + p.KVH + h) * REC_D + d];
         kw[e] = (float)p.k_norm[d];
       }
 #pragma unroll
@@ -361,7 +380,7 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
       fvq[f] = vq;
       fks[f] = ks;
       fvs[f] = vs;
-      fslot[f] = (pos % PAGE) * REC_KVH + hh;
+      fslot[f] = pos % PAGE;
       fpg[f] = pos / PAGE;
     }
   }
@@ -381,39 +400,33 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
   }
   // K operand rows: key block b, row n is key 8 (n / 4) + 4 b + n % 4, so the score lanes end up holding keys
   // 8 g .. 8 g + 7 of their row, the keys of their P^T operand.
-  const int kr0 = ((8 * (n >> 2) + (n & 3)) * REC_KVH + h) * REC_BYTES + 8 * g;
-  const int kr1 = kr0 + 4 * REC_KVH * REC_BYTES;
+  const int kr0 = (8 * (n >> 2) + (n & 3)) * LREC + 8 * g;
+  const int kr1 = kr0 + 4 * LREC;
 
-  auto step = [&](int k, const char* cur, char* nxt) {
-    if (k + 1 < nsteps)
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPW));
-    else
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __builtin_amdgcn_s_barrier();  // page k is in LDS; every wave is done with page k - 1 (its slot, vt, kvs)
-    if (k + 2 < nsteps) issue(k + 2, nxt);
+  auto step = [&](int k, char* cur, char* nxt) {
+    ring_barrier<LPW>();  // page k is in LDS; every wave is done with page k - 1 (its slot, vt, kvs)
+    issue(k + 2, paged ? __builtin_amdgcn_readfirstlane(sm_bt[min(k + 2, nsteps - 1)]) : pb + k + 2, nxt);
     // fresh records of page k into its LDS copy (stale in the pool), then a barrier
     if (fresh && p.a + p.M - 1 >= (pb + k) * PAGE && p.a < (pb + k + 1) * PAGE) {
 #pragma unroll
       for (int f = 0; f < FPW; ++f) {
         if (fpg[f] == pb + k && lane < 32) {
-          char* rec = const_cast<char*>(cur) + fslot[f] * REC_BYTES;
+          char* rec = cur + fslot[f] * LREC;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             rec[lane + 32 * e] = (char)((fkq[f] >> (8 * e)) & 255);
-            rec[REC_D + 4 + lane + 32 * e] = (char)((fvq[f] >> (8 * e)) & 255);
+            rec[LREC_V + lane + 32 * e] = (char)((fvq[f] >> (8 * e)) & 255);
           }
           if (lane == 0) {
-            *reinterpret_cast<float*>(rec + REC_D) = fks[f];
-            *reinterpret_cast<float*>(rec + 2 * REC_D + 4) = fvs[f];
+            *reinterpret_cast<float*>(rec + LREC_KS) = fks[f];
+            *reinterpret_cast<float*>(rec + LREC_VS) = fvs[f];
           }
         }
       }
-      __builtin_amdgcn_s_waitcnt(LGKMCNT0_IMM);
-      __builtin_amdgcn_s_barrier();
+      lds_barrier();
     }
     rec_expand<NT>(cur, vt, kvs);
-    __builtin_amdgcn_s_waitcnt(LGKMCNT0_IMM);
-    __builtin_amdgcn_s_barrier();
+    lds_barrier();
     const int page = pb + k;
     int64_t ka[2][4];
 #pragma unroll
@@ -421,8 +434,8 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
       ka[0][grp] = *reinterpret_cast<const int64_t*>(cur + kr0 + 32 * grp);
       ka[1][grp] = *reinterpret_cast<const int64_t*>(cur + kr1 + 32 * grp);
     }
-    const f32x4 ks0 = *reinterpret_cast<const f32x4*>(kvs + (h * 2) * PAGE + 8 * g);
-    const f32x4 ks1 = *reinterpret_cast<const f32x4*>(kvs + (h * 2) * PAGE + 8 * g + 4);
+    const f32x4 ks0 = *reinterpret_cast<const f32x4*>(kvs + 8 * g);
+    const f32x4 ks1 = *reinterpret_cast<const f32x4*>(kvs + 8 * g + 4);
     f32x4 sc[QB][2];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
@@ -488,8 +501,8 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
         }
       }
     }
-    const f32x4 vs0 = *reinterpret_cast<const f32x4*>(kvs + (h * 2 + 1) * PAGE + 8 * g);
-    const f32x4 vs1 = *reinterpret_cast<const f32x4*>(kvs + (h * 2 + 1) * PAGE + 8 * g + 4);
+    const f32x4 vs0 = *reinterpret_cast<const f32x4*>(kvs + PAGE + 8 * g);
+    const f32x4 vs1 = *reinterpret_cast<const f32x4*>(kvs + PAGE + 8 * g + 4);
     half8 pp[QB];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
@@ -506,7 +519,7 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
     // one V^T operand at a time, shared by the row blocks
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      const half8 vop = *reinterpret_cast<const half8*>(vt + (h * 8 + c) * VT_CHUNK + vt_slot(lane));
+      const half8 vop = *reinterpret_cast<const half8*>(vt + c * VT_CHUNK + vt_slot(lane));
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) o[qb][c] = mfma16x16x32(vop, pp[qb], o[qb][c]);
     }
@@ -523,8 +536,9 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
     for (int f = 0; f < FPW; ++f) {
       if (fpg[f] >= 0 && lane < 32) {
         const int phys = paged ? sm_bt[fpg[f] - pb] : fpg[f];
+        if ((uint64_t)(phys + 1) * REC_PAGE > p.k_bytes) continue;
         uint8_t* rec = reinterpret_cast<uint8_t*>(const_cast<_Float16*>(p.kp)) + (size_t)phys * REC_PAGE +
-                       (size_t)fslot[f] * REC_BYTES;
+                       ((size_t)fslot[f] * REC_KVH + h) * REC_BYTES;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           rec[lane + 32 * e] = (uint8_t)((fkq[f] >> (8 * e)) & 255);
@@ -564,9 +578,9 @@ __global__ __launch_bounds__(REC_KVH * NRG * 64) void verify_attn_rec_kernel(Att
 #undef DSPARK_LDSP
 
 // ---------------------------------------------------------------- host side
-// One wave per (KV head, 16-row block): up to 4 row blocks per head (64 rows: 16 tokens at 4 query heads per KV head;
-// the reference verifies at most 9). Measured alternatives at 128k keys: two row blocks per wave in 8 waves (the 36 rows
-// of 9 tokens padded to 64) 52.0 against 45.1 us; one wave per head with all its row blocks 52.8 us.
+// One wave per 16-row block: up to 4 row blocks per head (64 rows: 16 tokens at 4 query heads per KV head; the reference
+// verifies at most 9), and at least two waves to share a page's loads and expansion (1 token at 256 / 4096 / 131072 keys:
+// one wave 54.5 / 73.6 / 233.5 us for six layers, two 49.0 / 64.2 / 231.9).
 void attn_rec_plan(AttnParams& p, int cus) {
   const int rows = p.G * p.M;
   const int nblk = (rows + 15) / 16;
@@ -581,18 +595,22 @@ void attn_rec_plan(AttnParams& p, int cus) {
   p.lds = 2;
   p.nrb = nblk;
   p.qb = 1;
-  p.nrg = nblk;
+  p.nrg = std::max(nblk, 2);
   p.pl = p.ppl = p.lpw = 1;
   p.RG = 1;
   p.QB = 1;
   p.R = 16 * nblk;
   p.OCC = 1;
   int S = p.S;
-  // One workgroup per CU (the LDS ring). A split costs ~8 us before its first page and ~1.9 us per page, so up to 96
-  // pages every page gets its own split (the merge keeps its 8-lane form); beyond, two pages or more per split (4096
-  // keys: 129 one-page splits took 16.8 us per layer with the merge, 65 two-page splits 16.2; 1024 keys 12.9 against
-  // 14.8; reference-geometry rounds 1.448 -> 1.428 ms at 1k).
-  if (S <= 0) S = p.npages <= 96 ? p.npages : std::min(cus, (p.npages + 1) / 2);
+  // A split costs ~5 us beside its pages, and its partials (8 KB per token) are written and read back, so a row block more
+  // asks for longer splits: 3, 5 or 8 pages for 1, 2 or more row blocks. But never fewer splits than give each CU a
+  // workgroup (8 tokens, 4096 / 8192 keys: 43 / 52 splits 73.6 / 87.3 us for six layers, 65 / 86 splits 76.3 / 90.1), and no
+  // more than the workgroups resident at once (three per CU; four measured better for one row block: 131072 keys, 256 /
+  // 192 splits: 4 tokens 238 / 269 us; 16 tokens at 32771 keys, 129 / 171 splits 158 / 182 us).
+  if (S <= 0) {
+    const int per = nblk == 1 ? 3 : nblk == 2 ? 5 : 8, most = nblk == 1 ? 4 : 3;
+    S = std::min(std::max((p.npages + per - 1) / per, cus / REC_KVH), most * cus / REC_KVH);
+  }
   S = std::max(S, (p.npages + REC_BT_MAX - 1) / REC_BT_MAX);
   S = std::max(1, std::min(S, std::min(ATTN_REC_MAX_SPLITS, p.npages)));
   p.pps = (p.npages + S - 1) / S;
@@ -602,12 +620,11 @@ void attn_rec_plan(AttnParams& p, int cus) {
 int attn_rec_launch(AttnParams& p, int phases, hipStream_t s) {
   if (phases & 1) {
     if (p.KVH != REC_KVH || p.pps > REC_BT_MAX || p.nrb < 1 || p.nrb > 4 || p.qb * p.nrg < p.nrb) return DSPARK_EUNSUPPORTED;
-    const dim3 grid(p.S);
+    const dim3 grid((p.S + 7) / 8 * 8 * REC_KVH);
     switch (p.qb * 10 + p.nrg) {
-      case 11: hipLaunchKernelGGL((verify_attn_rec_kernel<1, 1>), grid, dim3(REC_KVH * 1 * 64), 0, s, p); break;
-      case 12: hipLaunchKernelGGL((verify_attn_rec_kernel<1, 2>), grid, dim3(REC_KVH * 2 * 64), 0, s, p); break;
-      case 13: hipLaunchKernelGGL((verify_attn_rec_kernel<1, 3>), grid, dim3(REC_KVH * 3 * 64), 0, s, p); break;
-      case 14: hipLaunchKernelGGL((verify_attn_rec_kernel<1, 4>), grid, dim3(REC_KVH * 4 * 64), 0, s, p); break;
+      case 12: hipLaunchKernelGGL((verify_attn_rec_kernel<1, 2>), grid, dim3(2 * 64), 0, s, p); break;
+      case 13: hipLaunchKernelGGL((verify_attn_rec_kernel<1, 3>), grid, dim3(3 * 64), 0, s, p); break;
+      case 14: hipLaunchKernelGGL((verify_attn_rec_kernel<1, 4>), grid, dim3(4 * 64), 0, s, p); break;
       default: return DSPARK_EUNSUPPORTED;
     }
     const hipError_t e = hipGetLastError();

@@ -71,6 +71,9 @@ __device__ __forceinline__ void ring_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Every wave's LDS accesses done, none moved across (loads from memory stay in flight).
+__device__ __forceinline__ void lds_barrier() { ring_barrier<63>(); }
+
 // Butterfly over a whole wave without the LDS unit (a shuffle there costs about 100 cycles a level): level by level each
 // lane's value is combined with lane ^ 32's and lane ^ 16's by the half-wave swaps, then with lane ^ 8's, ^ 4's, ^ 2's
 // and ^ 1's by row rotations -- after a level the values repeat with half the period, so that a rotation by 4 in a row of
