@@ -25,6 +25,15 @@
 #include "dspark_internal.h"
 #include "attn_range.h"
 
+// The launch indexes and rsqrt by the compiler's builtins: this file's floating-point flags differ from the device
+// library's, whose functions (threadIdx, blockIdx, rsqrtf) are then called, not inlined -- a call per use, with a call's
+// registers, before the first load. Without them, without divisions and with the merge's loads as buffer offsets: six
+// layers with their merges at 1001 keys (D 128, 8 tokens) 56.1 -> 53.5 us, at 32768 (D 64, 16 tokens) 111.9 -> 109.9.
+#define TID __builtin_amdgcn_workitem_id_x()
+#define WG_X __builtin_amdgcn_workgroup_id_x()
+#define WG_Y __builtin_amdgcn_workgroup_id_y()
+#define WG_Z __builtin_amdgcn_workgroup_id_z()
+
 namespace dspark {
 
 constexpr float TAU = 8.f;        // lazy-rescale slack in log2 units
@@ -122,7 +131,7 @@ __device__ __forceinline__ void page_prep(const AttnParams& p, int lpage, int ro
     for (int qb = 0; qb < QB; ++qb) {
       // Visible keys of the lane's row (token t = row / G; padding rows act as the last token): start and the window
       // bound the context keys only (dspark.hip:1308-1312, 2006-2012), the block's own keys are visible up to t.
-      const int t = min((row0 + 16 * qb + (lane & 15)) / p.G, p.M - 1);
+      const int t = min(div_by(row0 + 16 * qb + (lane & 15), p.g_div), p.M - 1);
       const int lo = min(p.a, max(p.start, p.window > 0 ? p.a + t - p.window + 1 : 0));
       const int hi = p.causal ? p.a + t : p.a + p.M - 1;
 #pragma unroll
@@ -187,12 +196,12 @@ template <int D, int QB, int PF, int OCC, bool QLDS>
 __global__ __launch_bounds__(256, OCC) void verify_attn_kernel(AttnParams p) {
   if (p.st && !attn_state_range(p)) return;
   constexpr int R = 16 * QB;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: page indices stay scalar
+  const int lane = TID & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(TID >> 6);  // uniform: page indices stay scalar
   const int n = lane & 15, g = lane >> 4;
   // Workgroups are dealt to the 8 XCDs round-robin (id % 8). Row groups of one (head, split) read the same pages, so
   // they take ids 8 apart inside a chunk of 8*RG: same XCD (shared L2), dispatched together.
-  const int bid = blockIdx.x;
+  const int bid = WG_X;
   const int chunk = bid / (8 * p.RG), within = bid % (8 * p.RG);
   const int rg = within / 8;
   const int unit = chunk * 8 + within % 8;
@@ -215,7 +224,7 @@ __global__ __launch_bounds__(256, OCC) void verify_attn_kernel(AttnParams p) {
     return q;
   };
   if constexpr (QLDS) {
-    for (int e = threadIdx.x; e < QB * (D / 32) * 64; e += 256) q_lds[e] = q_operand(e / ((D / 32) * 64), (e / 64) % (D / 32), e % 64);
+    for (int e = TID; e < QB * (D / 32) * 64; e += 256) q_lds[e] = q_operand(e / ((D / 32) * 64), (e / 64) % (D / 32), e % 64);
     qf.lds = q_lds;
     __syncthreads();
   } else {
@@ -309,11 +318,11 @@ __global__ __launch_bounds__(256, OCC) void verify_attn_kernel(AttnParams p) {
   // row-major partials: row r of this split at ((hr R + r) S + split)
   const size_t row0 = ((size_t)h * p.RG + rg) * R * p.S + split;
   f32x4* dst = reinterpret_cast<f32x4*>(p.part_acc) + row0 * (D / 4);
-  for (int e = threadIdx.x; e < R * D / 4; e += 256) {
+  for (int e = TID; e < R * D / 4; e += 256) {
     const int r = e / (D / 4), c4 = e % (D / 4);
     dst[(size_t)r * p.S * (D / 4) + c4] = sm_o[0][r][c4] + sm_o[1][r][c4];
   }
-  for (int r = threadIdx.x; r < R; r += 256) {
+  for (int r = TID; r < R; r += 256) {
     const float mx = fmaxf(fmaxf(sm_m[0][r], sm_m[1][r]), fmaxf(sm_m[2][r], sm_m[3][r]));
     const float L = (fast_exp2(sm_m[1][r] - mx) * sm_l[1][r] + fast_exp2(sm_m[0][r] - mx) * sm_l[0][r]) +
                     (fast_exp2(sm_m[3][r] - mx) * sm_l[3][r] + fast_exp2(sm_m[2][r] - mx) * sm_l[2][r]);
@@ -381,11 +390,13 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
   // later, with the arguments the block-table loads need, its miss would delay them.
   if constexpr (FR) asm volatile("" ::"s"(p.rope));
   if (p.st && !attn_state_range(p)) return;
-  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = TID & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(TID >> 6);
   const int NRB = p.nrb, NRG = p.nrg, NW = NRG * PL;
-  const int rg = wave % NRG, pl = wave / NRG;
-  const int h = blockIdx.x / p.S, split = blockIdx.x % p.S;
+  static_assert(PL <= 4, "page lanes by comparison");
+  const int pl = (PL > 1 && wave >= NRG) + (PL > 2 && wave >= 2 * NRG) + (PL > 3 && wave >= 3 * NRG);
+  const int rg = wave - pl * NRG;
+  const int h = WG_Y, split = WG_X;
   const int R = NRB * 16;
 
   QOps<D, QB, false> qf;
@@ -412,7 +423,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
   // vector load (the direct-to-LDS loads count as possible clobbers), and its wait would drain the pages in flight.
   const bool paged = p.bt != nullptr;
   if (paged) {
-    for (int i = threadIdx.x; i < pe - pb; i += NW * 64) sm_bt[i] = ldg(p.bt + pb + i);
+    for (int i = TID; i < pe - pb; i += NW * 64) sm_bt[i] = ldg(p.bt + pb + i);
     __syncthreads();
   }
 
@@ -509,7 +520,8 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const int r = min((rg * QB + qb) * 16 + n, p.G * p.M - 1);
-      const float* qr = p.mix + (size_t)(r / p.G) * p.mix_row + (size_t)(h * p.G + r % p.G) * D + 8 * g;
+      const int t = div_by(r, p.g_div);
+      const float* qr = p.mix + (size_t)t * p.mix_row + (size_t)(h * p.G + r - t * p.G) * D + 8 * g;
 #pragma unroll
       for (int s = 0; s < D / 32; ++s) {
         fq[qb][s][0] = ldg(reinterpret_cast<const f32x4*>(qr + 32 * s));
@@ -540,7 +552,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
 #pragma unroll
     for (int s = 0; s < D / 64; ++s) {
       const int r = min(rg * QB * 16 + n, p.G * p.M - 1);
-      const _Float16* rt = p.rope + (size_t)(p.a + r / p.G) * D + 32 * s + 8 * g;
+      const _Float16* rt = p.rope + (size_t)(p.a + div_by(r, p.g_div)) * D + 32 * s + 8 * g;
       fqc[s] = ldg(reinterpret_cast<const half8*>(rt));
       fqs[s] = ldg(reinterpret_cast<const half8*>(rt + D / 2));
     }
@@ -552,7 +564,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
     for (int qb = 0; qb < QB; ++qb) {
       const int rb = rg * QB + qb;
       const int r = min(rb * 16 + n, p.G * p.M - 1);
-      const int t = r / p.G, qh = h * p.G + r % p.G;
+      const int t = div_by(r, p.g_div), qh = h * p.G + r - t * p.G;
 #pragma unroll
       for (int s = 0; s < D / 32; ++s)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, DSPARK_LDSP(q_lds + (rb * (D / 32) + s) * 1024), 16,
@@ -605,7 +617,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
         }
       ss += __shfl_xor(ss, 16);
       ss += __shfl_xor(ss, 32);
-      const float inv = rsqrtf(ss / D + p.eps);
+      const float inv = __builtin_amdgcn_rsqf(ss / D + p.eps);
 #pragma unroll
       for (int s = 0; s < D / 32; ++s)
 #pragma unroll
@@ -635,7 +647,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
       for (int e = 0; e < NE; ++e) ss += fk[e] * fk[e];
       ss = (lane < 32) ? ss : 0.f;
       ss = wave_sum(ss);
-      const float inv = rsqrtf(ss / D + p.eps);
+      const float inv = __builtin_amdgcn_rsqf(ss / D + p.eps);
       float r[NE];
 #pragma unroll
       for (int e = 0; e < NE; ++e) r[e] = fk[e] * inv * (float)fkw[e];
@@ -768,7 +780,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
 // 64 / (D / 4) whole splits of the row, contiguous), and merges them as a log-sum-exp (m = max, l = sum f_s l_s,
 // acc = sum f_s acc_s, f_s = exp2(m_s - m)); the split lanes of a wave then merge pairwise in a fixed xor tree and the
 // waves in wave order through LDS, so outputs are bit-identical run to run. o = acc / l (0 when nothing was visible),
-// times the optional sigmoid gate, stored fp16 and/or fp32. blockIdx = (row, KV head x row group); rows past G M (padding
+// times the optional sigmoid gate, stored fp16 and/or fp32. blockIdx = (row, KV head, row group); rows past G M (padding
 // of the last row block, never stored by the split kernels) store nothing. Measured on MI355X, graph-replayed with the
 // partials in HBM: 256 splits at D 128 6.8 us (18.7 with the split-major layout and 32 lanes per output quad, whose
 // every load touched 32 cache lines), 64 splits 3.6 (4.9), C2's 24 splits at D 64 2.8 with 4 split lanes, one wave
@@ -781,23 +793,26 @@ __global__ __launch_bounds__(SL * D / 4) void attn_combine_kernel(AttnParams p) 
   static_assert(NT % 64 == 0 && 64 % Q == 0, "whole waves of whole rows");
   __shared__ f32x4 s_acc[W > 1 ? W - 1 : 1][Q];
   __shared__ f32x2 s_ml[W > 1 ? W - 1 : 1][Q];
-  const int hr = blockIdx.y, h = hr / p.RG, rg = hr % p.RG, r = blockIdx.x;
+  const int h = WG_Y, rg = WG_Z, hr = h * p.RG + rg, r = WG_X;
   const int row = rg * p.R + r;
   // Padding rows of the last row group (row >= G M, the same for the whole workgroup) load their partials (inside the
   // workspace) and store nothing: returning before the loads would put the kernel arguments the loads need behind the
   // test's own, one more dependent round trip for every row.
   const bool live = row < p.G * p.M;
-  const int run = run_flag_load(p.st);  // tested once the partial loads are in flight
+  const int q = TID % Q, j = TID / Q;
+  // (32-bit products: a 64-bit one is a vector operation, and its buffer a loop over the lanes per load)
+  const size_t base = (size_t)(((uint32_t)hr * (uint32_t)p.R + (uint32_t)r) * (uint32_t)p.S);
+  // The row's partials as two buffers, so that a load is its 32-bit offset (splits past S read nothing): the first loads
+  // leave some 60 instructions into the kernel, not 140 to 320.
+  const __amdgpu_buffer_rsrc_t racc = __builtin_amdgcn_make_buffer_rsrc((void*)(p.part_acc + base * D), (short)0,
+                                                                        p.S * D * (int)sizeof(float), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rml =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(p.part_ml + base), (short)0, p.S * (int)sizeof(f32x2), 0x00020000);
+  int run;
   // The gate word is loaded with the partials (a zero-length buffer when there is no gate: the load returns 0).
   const int rowc = min(row, p.G * p.M - 1);
-  const int t = rowc / p.G, qh = h * p.G + rowc % p.G;
-  const int gstride = p.gate_stride > 0 ? p.gate_stride : p.QH;
-  const __amdgpu_buffer_rsrc_t rgate = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)p.gate, (short)0, p.gate ? (int)((size_t)p.M * gstride * sizeof(float)) : 0, 0x00020000);
-  const float gv = __builtin_bit_cast(
-      float, __builtin_amdgcn_raw_buffer_load_b32(rgate, (int)(((size_t)t * gstride + qh) * sizeof(float)), 0, 0));
-  const int q = threadIdx.x % Q, j = threadIdx.x / Q;
-  const size_t base = ((size_t)hr * p.R + r) * p.S;
+  const int t = div_by(rowc, p.g_div), qh = h * p.G + rowc - t * p.G;
+  float gv;
   float m = -INFINITY, l = 0.f;
   f32x4 acc = {0, 0, 0, 0};
   // Batches of SL x PER splits; the first is outside the loop (a loop head's wait, counted for the back edge, would hold
@@ -808,10 +823,21 @@ __global__ __launch_bounds__(SL * D / 4) void attn_combine_kernel(AttnParams p) 
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int sp = b0 + j + SL * i;
-      const bool ok = sp < p.S;
-      ml[i] = ok ? ldg(p.part_ml + base + sp) : f32x2{-INFINITY, 0.f};
-      av[i] = ok ? ldg(reinterpret_cast<const f32x4*>(p.part_acc + (base + sp) * D) + q) : f32x4{0, 0, 0, 0};
+      ml[i] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rml, sp * (int)sizeof(f32x2), 0, 0));
+      av[i] = __builtin_bit_cast(f32x4,
+                                 __builtin_amdgcn_raw_buffer_load_b128(racc, (sp * D + 4 * q) * (int)sizeof(float), 0, 0));
     }
+    if (b0 == 0) {
+      run = run_flag_load(p.st);
+      const int gstride = p.gate_stride > 0 ? p.gate_stride : p.QH;
+      const __amdgpu_buffer_rsrc_t rgate = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)p.gate, (short)0, p.gate ? p.M * gstride * (int)sizeof(float) : 0, 0x00020000);
+      gv = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(rgate, (int)(((size_t)t * gstride + qh) * sizeof(float)), 0, 0));
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (b0 + j + SL * i >= p.S) ml[i][0] = -INFINITY;
     if (!run_flag_set(run) || !live) {  // a stopped round or a padding row writes nothing (the whole workgroup)
       __builtin_amdgcn_s_waitcnt(0);
       return false;
@@ -852,7 +878,7 @@ __global__ __launch_bounds__(SL * D / 4) void attn_combine_kernel(AttnParams p) 
     for (int i = 0; i < 4; ++i) ak[i] = __shfl_xor(acc[i], off);
     fold(__shfl_xor(m, off), __shfl_xor(l, off), ak);
   }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = TID >> 6, lane = TID & 63;
   if constexpr (W > 1) {
     if (wave > 0 && lane < Q) {
       s_acc[wave - 1][q] = acc;
@@ -909,7 +935,7 @@ __global__ __launch_bounds__(256) void kv_write_kernel(const _Float16* k, const 
   constexpr int VROW = 20;       // dwords of a V^T row in LDS (16 pairs + padding)
   constexpr int NK = 32 * P / 256, NV = (16 * P + 255) / 256;
   __shared__ __attribute__((aligned(16))) uint32_t vt[D * VROW];
-  const int h = blockIdx.x % KVH, lp = pos0 / PAGE + (int)(blockIdx.x / KVH);
+  const int h = WG_X % KVH, lp = pos0 / PAGE + (int)(WG_X / KVH);
   const int phys = bt ? bt[lp] : lp;
   if (phys < 0 || phys >= kv_pages) return;  // a table entry outside the pools: its rows are not written
   const int base = lp * PAGE - pos0;         // the row of slot 0 (negative on the first page)
@@ -923,18 +949,18 @@ __global__ __launch_bounds__(256) void kv_write_kernel(const _Float16* k, const 
   u32x4 kv[NK], va[NV], vb[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int e = min((int)threadIdx.x + 256 * i, 16 * P - 1), pair = e / P, pc = e % P;
+    const int e = min((int)TID + 256 * i, 16 * P - 1), pair = e / P, pc = e % P;
     va[i] = piece(vr, 2 * pair, pc);
     vb[i] = piece(vr, 2 * pair + 1, pc);
   }
 #pragma unroll
   for (int i = 0; i < NK; ++i) {
-    const int e = threadIdx.x + 256 * i;
+    const int e = TID + 256 * i;
     kv[i] = piece(kr, e / P, e % P);
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int e = threadIdx.x + 256 * i, pair = e / P, pc = e % P;
+    const int e = TID + 256 * i, pair = e / P, pc = e % P;
     if (e < 16 * P) {
       // (the row's quads of pairs permuted by its piece, so that the 8 pieces of a slot fall on different banks)
       uint32_t* row = vt + 8 * pc * VROW + (((pair >> 2) ^ (pc & 3)) << 2) + (pair & 3);
@@ -950,7 +976,7 @@ __global__ __launch_bounds__(256) void kv_write_kernel(const _Float16* k, const 
   u32x4* kd = reinterpret_cast<u32x4*>(kp + ((size_t)phys * KVH + h) * (PAGE * D));
 #pragma unroll
   for (int i = 0; i < NK; ++i) {
-    const int e = threadIdx.x + 256 * i, slot = e / P, pc = e % P;
+    const int e = TID + 256 * i, slot = e / P, pc = e % P;
     if (slot >= s0 && slot < s1)
       kd[(((slot >> 2) & 1) * (D / 32) + (pc >> 2)) * 64 + 4 * (slot >> 3) + (slot & 3) + 16 * (pc & 3)] = kv[i];
   }
@@ -958,7 +984,7 @@ __global__ __launch_bounds__(256) void kv_write_kernel(const _Float16* k, const 
   _Float16* vd = vp + ((size_t)phys * KVH + h) * (D * PAGE);
 #pragma unroll
   for (int i = 0; i < D * 4 / 256; ++i) {
-    const int e = threadIdx.x + 256 * i, d = e >> 2, q = e & 3;
+    const int e = TID + 256 * i, d = e >> 2, q = e & 3;
     const u32x4 w = *reinterpret_cast<const u32x4*>(vt + d * VROW + ((q ^ ((d >> 3) & 3)) << 2));
     if (8 * q >= s0 && 8 * q + 8 <= s1) {
       *reinterpret_cast<u32x4*>(vd + d * PAGE + 8 * q) = w;
@@ -1019,13 +1045,13 @@ static int launch_lds(const AttnParams& p, hipStream_t s) {
   if constexpr (QB == 1 && D == 64) {
     if (p.mix) {  // a fresh block: at most one block token per wave
       if (p.M > p.nrg * PL) return DSPARK_EUNSUPPORTED;
-      hipLaunchKernelGGL((verify_attn_lds_kernel<D, QB, PL, PPL, LPW, MAXW, true>), dim3(p.KVH * p.S),
+      hipLaunchKernelGGL((verify_attn_lds_kernel<D, QB, PL, PPL, LPW, MAXW, true>), dim3(p.S, p.KVH),
                          dim3(p.nrg * PL * 64), 0, s, p);
       return 0;
     }
   }
   if (p.mix) return DSPARK_EUNSUPPORTED;
-  hipLaunchKernelGGL((verify_attn_lds_kernel<D, QB, PL, PPL, LPW, MAXW>), dim3(p.KVH * p.S), dim3(p.nrg * PL * 64), 0, s,
+  hipLaunchKernelGGL((verify_attn_lds_kernel<D, QB, PL, PPL, LPW, MAXW>), dim3(p.S, p.KVH), dim3(p.nrg * PL * 64), 0, s,
                      p);
   return 0;
 }
@@ -1203,13 +1229,15 @@ static int launch_split(const AttnParams& p, int D, hipStream_t s) {
 }
 
 int attn_launch(AttnParams& p, int D, int phases, hipStream_t s) {
+  p.s_div = div_magic((uint32_t)p.S);
+  p.g_div = div_magic((uint32_t)p.G);
   if (phases & 1) {
     const int rc = launch_split(p, D, s);
     if (rc) return rc;
   }
   if (phases & 2) {
     const bool wide = p.S > 96;  // 16 split lanes per row, else 8 (4 at D = 64 up to 32 splits: one wave per row)
-    const dim3 grid(p.R, p.KVH * p.RG);
+    const dim3 grid(p.R, p.KVH, p.RG);
     if (D == 64 && p.S <= 32)
       hipLaunchKernelGGL((attn_combine_kernel<64, 4>), grid, dim3(4 * 16), 0, s, p);
     else if (D == 64 && !wide)

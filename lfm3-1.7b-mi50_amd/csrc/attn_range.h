@@ -25,14 +25,14 @@ __device__ inline void attn_range(AttnParams& p, int a, int ctx_lo) {
   p.full_hi = p.causal ? a : hi_last;
   p.page0 = lo0 / PAGE;
   p.npages = hi_last / PAGE - p.page0 + 1;
-  p.pps = (p.npages + p.S - 1) / p.S;
+  p.pps = div_by(p.npages + p.S - 1, p.s_div);  // (a pool under 2 GiB: fewer than 2^20 pages, S at most 256)
 }
 
 // A key-split kernel's prologue with a State: run, a and ctx_lo read in one round trip (scalar loads of one line; the
 // empty asm takes all three before the run test, which would otherwise put the other two behind it). Returns false
 // when the round is stopped.
 __device__ inline bool attn_state_range(AttnParams& p) {
-  const int run = p.st->run, a = p.st->a, lo = p.st->ctx_lo;
+  const int run = ldc(&p.st->run), a = ldc(&p.st->a), lo = ldc(&p.st->ctx_lo);
   asm volatile("" ::"s"(run), "s"(a), "s"(lo));
   if (run == 0) return false;
   attn_range(p, a, lo);

@@ -207,10 +207,13 @@ __global__ __launch_bounds__(NRG * 64, NRG <= 2 ? 2 : 3) void verify_attn_rec_ke
   const bool paged = p.bt != nullptr;
   // The first two pages' table entries by scalar loads, so that their loads wait for nothing else; all of them to LDS
   // behind those loads, for the steps.
-  int first[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) first[i] = paged && nsteps > 0 ? (int)min((uint32_t)p.bt[pb + min(i, nsteps - 1)], REC_NO_PAGE) : pb + i;
-  const int my_bt = paged && nsteps > 0 ? ldg(p.bt + pb + min((int)threadIdx.x, nsteps - 1)) : 0;
+  int first[2] = {pb, pb + 1}, my_bt = 0;
+  if (paged && nsteps > 0) {
+    const int b0 = ldc(p.bt + pb), b1 = ldc(p.bt + min(pb + 1, pe - 1));
+    my_bt = ldg(p.bt + pb + min((int)threadIdx.x, nsteps - 1));
+    first[0] = (int)min((uint32_t)b0, REC_NO_PAGE);
+    first[1] = (int)min((uint32_t)b1, REC_NO_PAGE);
+  }
   if (paged)
     for (int i = (int)threadIdx.x + NT; i < nsteps; i += NT) sm_bt[i] = (uint16_t)min((uint32_t)ldg(p.bt + pb + i), REC_NO_PAGE);
 
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(NRG * 64, NRG <= 2 ? 2 : 3) void verify_attn_rec_ke
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const int r = min((rg * QB + qb) * 16 + n, p.G * p.M - 1);
-      const int t = r / p.G, qh = h * p.G + r % p.G;
+      const int t = div_by(r, p.g_div), qh = h * p.G + r - t * p.G;
       const _Float16* qr = p.q + ((size_t)t * p.QH + qh) * REC_D + 8 * g;
 #pragma unroll
       for (int grp = 0; grp < 4; ++grp) qraw[qb][grp] = ldg(reinterpret_cast<const u32x4*>(qr + 32 * grp));
@@ -267,7 +270,7 @@ __global__ __launch_bounds__(NRG * 64, NRG <= 2 ? 2 : 3) void verify_attn_rec_ke
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const int r = min((rg * QB + qb) * 16 + n, p.G * p.M - 1);
-      const int t = r / p.G, qh = h * p.G + r % p.G;
+      const int t = div_by(r, p.g_div), qh = h * p.G + r - t * p.G;
       const float* qr = p.mix + (size_t)t * p.mix_row + (size_t)qh * REC_D + 8 * g;
       const _Float16* rt = p.rope + (size_t)(p.a + t) * REC_D + 8 * g;
       float x[4][8];
@@ -461,7 +464,7 @@ __global__ __launch_bounds__(NRG * 64, NRG <= 2 ? 2 : 3) void verify_attn_rec_ke
     if (base < p.full_lo || base + PAGE - 1 > p.full_hi) {
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
-        const int t = min(((rg * QB + qb) * 16 + n) / p.G, p.M - 1);
+        const int t = min(div_by((rg * QB + qb) * 16 + n, p.g_div), p.M - 1);
         // start and the window bound the context keys only (dspark.hip:1308-1312, 2006-2012)
         const int lo = min(p.a, max(p.start, p.window > 0 ? p.a + t - p.window + 1 : 0));
         const int hi = p.causal ? p.a + t : p.a + p.M - 1;
@@ -618,6 +621,8 @@ void attn_rec_plan(AttnParams& p, int cus) {
 }
 
 int attn_rec_launch(AttnParams& p, int phases, hipStream_t s) {
+  p.s_div = div_magic((uint32_t)p.S);
+  p.g_div = div_magic((uint32_t)p.G);
   if (phases & 1) {
     if (p.KVH != REC_KVH || p.pps > REC_BT_MAX || p.nrb < 1 || p.nrb > 4 || p.qb * p.nrg < p.nrb) return DSPARK_EUNSUPPORTED;
     const dim3 grid((p.S + 7) / 8 * 8 * REC_KVH);

@@ -41,6 +41,19 @@ __device__ __forceinline__ half8 i8x8_to_half8(uint32_t w0, uint32_t w1) {
   return h - bias;
 }
 
+// x / d by one multiplication: div_magic(d) = ceil(2^32 / d), exact for x d < 2^32 (0 stands for d = 1). A division by a
+// run-time value is some 20 dependent instructions, most of them before a kernel's first load.
+inline uint32_t div_magic(uint32_t d) { return d > 1 ? (uint32_t)((0x100000000ull + d - 1) / d) : 0u; }
+__device__ __forceinline__ int div_by(int x, uint32_t magic) { return magic ? (int)(((uint64_t)(uint32_t)x * magic) >> 32) : x; }
+
+// A wave-uniform word that nothing writes while the kernel runs, by a scalar load (a plain load becomes a vector load in
+// kernels where the compiler sees a store that might reach it).
+template <typename T>
+__device__ __forceinline__ T ldc(const T* p) {
+  typedef __attribute__((address_space(4))) const T CT;
+  return *(CT*)(uintptr_t)p;
+}
+
 template <typename T>
 __device__ __forceinline__ T ldg(const T* p) {
   typedef __attribute__((address_space(1))) const T GT;

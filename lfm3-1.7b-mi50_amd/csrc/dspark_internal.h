@@ -17,6 +17,7 @@ constexpr int CONV_RING = 128;  // conv history positions kept per layer (>= max
 struct AttnParams {
   const struct ::dspark_state* st;  // when set: a (and the drafter's ctx_lo) come from the State at run time
   int drafter;                      // with st: start = max(ctx_lo, a - window), no per-token window
+  uint32_t s_div;                   // div_magic of S and of G (set at launch)
   const _Float16* q;
   const _Float16* kp;
   const _Float16* vp;
@@ -30,6 +31,7 @@ struct AttnParams {
   // them as it loads them) and out_sc their scales, piece c / 16 of output column c = qh D + d at t out_sc_row + c / 16
   float* out_sc;
   int out_sc_row;
+  uint32_t g_div;
   const float* gate;
   int out_op;                 // > 0: out16 in the verify GEMM's X operand order with out_op token blocks
   int M, QH, KVH, G;
@@ -179,7 +181,7 @@ int attn_launch(AttnParams& p, int D, int phases, hipStream_t s);
 int kv_write_launch(const void* k, const void* v, int64_t row_stride, void* kp, void* vp, const int32_t* bt,
                     int64_t kv_pages, int KVH, int D, int pos0, int n, hipStream_t s);
 
-// Verify attention over int8 K/V records (attn_rec.hip): D = 128, 4 KV heads, one workgroup per key split of all heads,
+// Verify attention over int8 K/V records (attn_rec.hip): D = 128, 4 KV heads, one workgroup per KV head and key split,
 // up to ATTN_REC_MAX_SPLITS splits (the merge takes any split count); same partial format and merge as the fp16 path
 // (the workspace size is attn_workspace_bytes(p, 128) of the planned p).
 constexpr int ATTN_REC_MAX_SPLITS = 256;
