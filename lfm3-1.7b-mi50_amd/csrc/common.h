@@ -117,6 +117,15 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
   }));
 }
+// The sum of each half of a wave, in every lane of the half (the bits of wave_sum with zeros in the other half).
+__device__ __forceinline__ float half_wave_sum(float v) {
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  v += __uint_as_float(row_ror<8>(__float_as_uint(v)));
+  v += __uint_as_float(row_ror<4>(__float_as_uint(v)));
+  v += __uint_as_float(row_ror<2>(__float_as_uint(v)));
+  return v + __uint_as_float(row_ror<1>(__float_as_uint(v)));
+}
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return wave_butterfly(v, [](uint32_t a, uint32_t b) { return max(a, b); });
 }

@@ -114,6 +114,8 @@ struct QkRopeBatch {
   int n;
 };
 int qkrope_batch_launch(const QkRopeBatch& b, hipStream_t s);
+// The same for whole prompts: K/V rows only (no q16, no records), positions from the State's context, page by page.
+int kvrope_pages_launch(const QkRopeBatch& b, hipStream_t s);
 
 struct MarkovParams {
   struct ::dspark_state* st;

@@ -549,7 +549,7 @@ int project_wide(dspark_engine* e, const _Float16* x_fc, int n, GemmWideParams f
     b.n = std::min(QKROPE_BATCH, d.draft_layers - j0);
     for (int j = 0; j < b.n; ++j)
       b.l[j] = qk_params(e, e->DL[j0 + j], e->proj_y + (size_t)(j0 + j) * kvrow, rows, false, true, n);
-    CK(qkrope_batch_launch(b, s));
+    CK(kvrope_pages_launch(b, s));
   }
   return 0;
 }

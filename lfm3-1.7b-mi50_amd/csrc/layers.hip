@@ -336,6 +336,94 @@ __global__ __launch_bounds__(256) void qkrope_kernel(QkRopeParams p) { qkrope_bo
 template <int D>
 __global__ __launch_bounds__(256) void qkrope_batch_kernel(QkRopeBatch b) { qkrope_body<D>(b.l[blockIdx.y]); }
 
+// The K/V rows of many positions (a prompt's context projection), page by page: workgroup (KV head, page, layer) of 4 waves,
+// a half-wave per position as above (lane l holds dims l + 32 e), 8 positions a wave, all their loads in flight at once. K
+// and V go to LDS in the order of their pages (V transposed, rows of 40 halves) and from there in 16-byte pieces. What
+// bounds it is the rows' bytes (fp32 in, fp16 out) and one chain of loads: the kernel above stores V 2 bytes at a time, 64
+// bytes apart. 2048 positions, 5 layers of 8 heads, D = 64: 37.5 -> 10.2 us (the
+// whole projection 231 -> 198; 17 to 182 positions 1 to 11% less too).
+template <int D>
+__global__ __launch_bounds__(256) void kvrope_pages_kernel(QkRopeBatch b) {
+  const QkRopeParams& p = b.l[blockIdx.z];
+  asm volatile("" ::"s"(p.st), "s"(p.eps), "s"(p.count_from_ctx));  // (one round trip, as above)
+  constexpr int NE = D / 32, NP = PAGE / 8, VROW = 40;
+  __shared__ __attribute__((aligned(16))) _Float16 kt[PAGE * D], vt[D * VROW];
+  const int run = ldc(&p.st->run), pos0 = ldc(&p.st->ctx_pos), count = min(ldc(&p.st->ctx_new), p.M);
+  const int kvh = blockIdx.x, lp = pos0 / PAGE + (int)blockIdx.y;
+  const int base = lp * PAGE - pos0;  // the row of slot 0 (negative on the first page)
+  const int s0 = max(0, -base), s1 = min(PAGE, count - base);
+  if (run == 0 || s1 <= s0) return;
+  const int phys = p.bt ? ldc(p.bt + lp) : lp;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
+  float v[NP][NE], vv[NP][NE], wn[NE];
+  _Float16 cs[NP][NE / 2], sn[NP][NE / 2];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int slot = wave * 8 + 2 * i + (lane >> 5);
+    const int t = base + min(max(slot, s0), s1 - 1);  // slots outside the range read a row inside it
+    const float* src = p.mix + (size_t)t * p.row + (size_t)kvh * D;
+    const _Float16* rt = p.rope + (size_t)(pos0 + t) * D;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      v[i][e] = ldg(src + l + 32 * e);
+      vv[i][e] = ldg(src + (size_t)p.KVH * D + l + 32 * e);
+    }
+#pragma unroll
+    for (int e = 0; e < NE / 2; ++e) {
+      cs[i][e] = ldg(rt + l + 32 * e);
+      sn[i][e] = ldg(rt + D / 2 + l + 32 * e);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) wn[e] = (float)ldg(p.k_norm + l + 32 * e);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int slot = wave * 8 + 2 * i + (lane >> 5);
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) ss += v[i][e] * v[i][e];
+    const float inv = rsqrtf(half_wave_sum(ss) / D + p.eps);
+    float r[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) r[e] = v[i][e] * inv * wn[e];
+#pragma unroll
+    for (int e = 0; e < NE / 2; ++e) {
+      if (l + 32 * e < p.rot) {
+        const float c = (float)cs[i][e], s = (float)sn[i][e];
+        const float x0 = r[e], x1 = r[e + NE / 2];
+        r[e] = x0 * c - x1 * s;
+        r[e + NE / 2] = x1 * c + x0 * s;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      kt[k_page_elem(slot, l + 32 * e, D)] = (_Float16)r[e];
+      vt[(l + 32 * e) * VROW + slot] = (_Float16)vv[i][e];
+    }
+  }
+  __syncthreads();
+  // K: piece e is key slot 8 (n / 4) + 4 b + n % 4 (k_page_elem), 8 of its dims
+  u32x4* kd = reinterpret_cast<u32x4*>(p.kp + ((size_t)phys * p.KVH + kvh) * (PAGE * D));
+#pragma unroll
+  for (int i = 0; i < PAGE * D / 8 / 256; ++i) {
+    const int e = threadIdx.x + 256 * i, n = e & 15, slot = 8 * (n >> 2) + 4 * ((e >> 6) / (D / 32)) + (n & 3);
+    if (slot >= s0 && slot < s1) kd[e] = reinterpret_cast<const u32x4*>(kt)[e];
+  }
+  _Float16* vd = p.vp + ((size_t)phys * p.KVH + kvh) * (D * PAGE);
+#pragma unroll
+  for (int i = 0; i < D * 4 / 256; ++i) {
+    const int e = threadIdx.x + 256 * i, d = e >> 2, q = e & 3;
+    const half8 w = *reinterpret_cast<const half8*>(vt + d * VROW + 8 * q);
+    if (8 * q >= s0 && 8 * q + 8 <= s1) {
+      *reinterpret_cast<half8*>(vd + d * PAGE + 8 * q) = w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (8 * q + j >= s0 && 8 * q + j < s1) vd[d * PAGE + 8 * q + j] = w[j];
+    }
+  }
+}
+
 // ---------------------------------------------------------------- drafter: Markov + confidence (markov_phase)
 // Step j (0-based) proposes draft j+1 from prev = (j == 0 ? anchor : the token of step j-1's argmax key):
 //   cap = min(max_drafts, block - 1, min(limit - a, budget - count) - 1); steps j >= cap do nothing;
@@ -702,6 +790,24 @@ int qkrope_launch(const QkRopeParams& p, hipStream_t s) {
     hipLaunchKernelGGL(qkrope_kernel<64>, dim3((tasks + 3) / 4), dim3(256), 0, s, p);
   else
     hipLaunchKernelGGL(qkrope_kernel<128>, dim3((tasks + 3) / 4), dim3(256), 0, s, p);
+  return (int)hipGetLastError();
+}
+
+int kvrope_pages_launch(const QkRopeBatch& b, hipStream_t s) {
+  if (b.n < 1 || b.n > QKROPE_BATCH) return DSPARK_EINVAL;
+  const QkRopeParams& p = b.l[0];
+  for (int j = 0; j < b.n; ++j) {
+    const QkRopeParams& o = b.l[j];
+    if (o.M != p.M || o.KVH != p.KVH || o.D != p.D || o.q16 || o.rec || !o.st || !o.pos_from_ctx || !o.count_from_ctx)
+      return DSPARK_EINVAL;
+  }
+  if (p.M < 1 || (p.D != 64 && p.D != 128)) return DSPARK_EINVAL;
+  const dim3 grid(p.KVH, (p.M + PAGE - 2) / PAGE + 1, b.n);  // (from any slot of the first page)
+  if (grid.y > 65535) return DSPARK_EINVAL;
+  if (p.D == 64)
+    hipLaunchKernelGGL(kvrope_pages_kernel<64>, grid, dim3(256), 0, s, b);
+  else
+    hipLaunchKernelGGL(kvrope_pages_kernel<128>, grid, dim3(256), 0, s, b);
   return (int)hipGetLastError();
 }
 
