@@ -608,10 +608,10 @@ void attn_rec_plan(AttnParams& p, int cus) {
   // A split costs ~5 us beside its pages, and its partials (8 KB per token) are written and read back, so a row block more
   // asks for longer splits: 3, 5 or 8 pages for 1, 2 or more row blocks. But never fewer splits than give each CU a
   // workgroup (8 tokens, 4096 / 8192 keys: 43 / 52 splits 73.6 / 87.3 us for six layers, 65 / 86 splits 76.3 / 90.1), and no
-  // more than the workgroups resident at once (three per CU; four measured better for one row block: 131072 keys, 256 /
-  // 192 splits: 4 tokens 238 / 269 us; 16 tokens at 32771 keys, 129 / 171 splits 158 / 182 us).
+  // more than three workgroups per CU, or four where that measured better (131072 keys, 256 / 192 splits: 4 tokens 238 / 269 us,
+  // 9 tokens 292 / 297; but 8 tokens at 65536 keys 185 / 174, 16 at 131072 352 / 346).
   if (S <= 0) {
-    const int per = nblk == 1 ? 3 : nblk == 2 ? 5 : 8, most = nblk == 1 ? 4 : 3;
+    const int per = nblk == 1 ? 3 : nblk == 2 ? 5 : 8, most = nblk == 1 || nblk == 3 ? 4 : 3;
     S = std::min(std::max((p.npages + per - 1) / per, cus / REC_KVH), most * cus / REC_KVH);
   }
   S = std::max(S, (p.npages + REC_BT_MAX - 1) / REC_BT_MAX);

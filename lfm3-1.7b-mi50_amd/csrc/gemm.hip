@@ -1687,8 +1687,10 @@ static bool gemm_plan_few(int M, int N, int K, bool gs, GemmPlan* pl) {
 // Streamed plans (row-major operands on 16-byte boundaries, whole 128-byte steps; others take the plans below). Tiles of 4
 // strips, or of 8 for int8 weights where the busiest CU then has no more strips (half the x traffic: 128000 x 2048 at 64
 // tokens 84 against 91 us, but 40000 rows 40.4 against 39.0; fp16 weights, whose x is half as much, 154 against 147 us at
-// 128000 rows). K over workgroups until every CU has one, at least 4 steps each. Group scales have no workspace and so no
-// split: below 128 tiles they stay with the K-sliced plans.
+// 128000 rows). K over workgroups until every CU has one, at least 4 steps each, for K past 4096 only: up to there callers' workspaces
+// are empty (the K-sliced plans need none), and past it none asks for more than those plans'. Without a split (shorter K, group
+// scales) int8 weights need enough tiles against the K-sliced plans, fewer the more tokens those read x for (K 2048, us, K-sliced /
+// streamed): 128 tiles 6.8 / 7.6 at 4 tokens, 7.5 / 7.6 at 9, 9.0 / 7.7 at 16; 96 tiles 11.9 / 10.3 at 33, 14.9 / 10.2 at 64; 192 tiles 10.2 / 8.4 at 4.
 static bool gemm_plan_stream(int M, int N, int K, bool i8, bool split, bool gs, GemmPlan* pl) {
   const int wb = i8 ? 1 : 2, strips = N / 16, steps = K * wb / 128;
   if ((size_t)K * wb % 128 || (size_t)N * K * wb >= (size_t)1 << 31 || (size_t)M * K * 2 >= (size_t)1 << 31) return false;
@@ -1696,9 +1698,9 @@ static bool gemm_plan_stream(int M, int N, int K, bool i8, bool split, bool gs, 
   const auto per_cu = [&](int rs) { return rs * ((strips + rs * GEMM_STREAM_WGS - 1) / (rs * GEMM_STREAM_WGS)); };
   const int rs = i8 && !gs && per_cu(8) <= per_cu(4) ? 8 : 4;
   const int tiles = (strips + rs - 1) / rs;
-  if (gs && tiles < GEMM_STREAM_WGS / 2) return false;  // (no workspace, no split)
   int ks = 1;
-  while (split && tiles * ks * 2 <= GEMM_STREAM_WGS && steps / (2 * ks) >= 4) ks *= 2;
+  while (split && K > 4096 && tiles * ks * 2 <= GEMM_STREAM_WGS && steps / (2 * ks) >= 4) ks *= 2;
+  if (i8 && ks == 1 && tiles < GEMM_STREAM_WGS * (M <= 10 ? 6 : M <= 32 ? 4 : 3) / 8) return false;
   const int spk = (steps + ks - 1) / ks;
   *pl = GemmPlan{};
   pl->stream = pl->wpg = rs;
