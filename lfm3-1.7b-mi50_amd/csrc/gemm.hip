@@ -4,11 +4,13 @@
 // Layout. C^T[rows][tokens] = W[rows][K] * X^T[K][tokens] with v_mfma_f32_16x16x32_f16: a wave streams a 16-row strip
 // of W (lane l: row l%16, 16 contiguous bytes per 64-column chunk), X^T comes from the same 16-byte pieces of the
 // token rows. int8 -> fp16 is exact: byte b (= q + 128) placed under 0x64 is the half 1024 + b, minus 1152 gives q
-// (v_perm_b32 + v_pk_add_f16 per two weights). Two kernels: the K-sliced kernel (up to 32 tokens) gives a workgroup
+// (v_perm_b32 + v_pk_add_f16 per two weights). Four kernels: row-major operands go to the streamed kernel (rings of
+// direct-to-LDS row pieces) or, few rows with group scales, to the few-row kernel, each where it measured faster; operands in
+// operand order, unaligned ones and the rest to the other two. The K-sliced kernel (up to 32 tokens) gives a workgroup
 // S strips and all of K, its S x KW waves each stream one range of K with every weight load in flight and add the
 // ranges in LDS in range order; the split kernel (any M <= 64) gives each workgroup a share of K and lets the last
 // workgroup of a row group to arrive add the split partials in split order (or a reduce kernel does). Weights are read
-// once per call for all tokens; both are HBM-bound (about 2*M flop per weight byte).
+// once per call for all tokens; all are HBM-bound (about 2*M flop per weight byte).
 // Reference: gemv_phase / unit_dot_r (dspark.hip:541-716), head_run<true> (2219-2318), markov argmax (2322-2366).
 #include <type_traits>
 
