@@ -27,10 +27,9 @@
 //
 // What bounds it: a workgroup's chain per page (wait, expand, barrier, products: ~1.1 us alone on its CU) and ~5 us before
 // and after its pages, so the work is split by head as well as by key range: four heads' workgroups in 40 KB of LDS each
-// share a CU and fill each other's waits, and the same number of workgroups leaves a quarter of the partials to merge.
-// Against one workgroup per split for all four heads (whole 33 KB pages, one workgroup a CU), six layers with their
-// merges: 8 tokens at 256 / 4096 / 32771 / 131072 keys 69.7 / 91.5 / 144.2 / 259.8 -> 53.2 / 70.9 / 128.4 / 246.5 us, 16
-// tokens 91.4 / 123.6 / 197.8 / 354.8 -> 57.0 / 80.2 / 158.4 / 340.4.
+// share a CU and fill each other's waits. Against one workgroup per split for all four heads (whole 33 KB pages, one
+// workgroup a CU), a layer with its merge, the same splits and bits: 8 tokens at 256 / 4096 / 32771 / 131072 keys 11.4 /
+// 14.8 / 24.5 / 44.0 -> 8.6 / 12.3 / 21.0 / 39.3 us, 16 tokens 15.0 / 20.4 / 33.9 / 59.6 -> 9.3 / 15.1 / 28.0 / 57.6.
 #include "common.h"
 #include "dspark.h"
 #include "dspark_internal.h"
@@ -583,7 +582,7 @@ __global__ __launch_bounds__(NRG * 64, NRG <= 2 ? 2 : 3) void verify_attn_rec_ke
 // ---------------------------------------------------------------- host side
 // One wave per 16-row block: up to 4 row blocks per head (64 rows: 16 tokens at 4 query heads per KV head; the reference
 // verifies at most 9), and at least two waves to share a page's loads and expansion (1 token at 256 / 4096 / 131072 keys:
-// one wave 54.5 / 73.6 / 233.5 us for six layers, two 49.0 / 64.2 / 231.9).
+// one wave 54.5 / 73.6 / 233.5 us for six layers, two 49.0 / 64.2 / 231.9, both in 9 / 43 / 256 splits).
 void attn_rec_plan(AttnParams& p, int cus) {
   const int rows = p.G * p.M;
   const int nblk = (rows + 15) / 16;
@@ -605,15 +604,12 @@ void attn_rec_plan(AttnParams& p, int cus) {
   p.R = 16 * nblk;
   p.OCC = 1;
   int S = p.S;
-  // A split costs ~5 us beside its pages, and its partials (8 KB per token) are written and read back, so a row block more
-  // asks for longer splits: 3, 5 or 8 pages for 1, 2 or more row blocks. But never fewer splits than give each CU a
-  // workgroup (8 tokens, 4096 / 8192 keys: 43 / 52 splits 73.6 / 87.3 us for six layers, 65 / 86 splits 76.3 / 90.1), and no
-  // more than three workgroups per CU, or four where that measured better (131072 keys, 256 / 192 splits: 4 tokens 238 / 269 us,
-  // 9 tokens 292 / 297; but 8 tokens at 65536 keys 185 / 174, 16 at 131072 352 / 346).
-  if (S <= 0) {
-    const int per = nblk == 1 ? 3 : nblk == 2 ? 5 : 8, most = nblk == 1 || nblk == 3 ? 4 : 3;
-    S = std::min(std::max((p.npages + per - 1) / per, cus / REC_KVH), most * cus / REC_KVH);
-  }
+  // One page per split up to 96 pages, then two or more, at most a split per CU. A row's P is rounded to fp16 under its
+  // split's running max, so the split count shows in an output's last bits: it depends on the range and the card alone, not
+  // on the number of tokens. (Longer splits with more row blocks leave fewer partials to merge but round differently; a
+  // layer with its merge at 4096 keys, 129 pages in 65 splits / 43 for 8 tokens or 64 for 16: 12.3 / 11.6 us at 8 tokens,
+  // 15.1 / 13.0 at 16; at 32771 keys, 205 / 171 splits: 21.0 / 20.3 and 28.0 / 25.7.)
+  if (S <= 0) S = p.npages <= 96 ? p.npages : std::min(cus, (p.npages + 1) / 2);
   S = std::max(S, (p.npages + REC_BT_MAX - 1) / REC_BT_MAX);
   S = std::max(1, std::min(S, std::min(ATTN_REC_MAX_SPLITS, p.npages)));
   p.pps = (p.npages + S - 1) / S;

@@ -111,8 +111,8 @@ def test_bounds_are_checked_on_the_host():
 
 
 def test_record_entry_points_check_their_arguments():
-    """The int8-record path: workspace sizes of the reference geometry (one key split per workgroup over all four KV
-    heads, the fp16 path's partial layout), and refusals before any launch (D, KVH, rows, a V pool, pools of 2 GiB,
+    """The int8-record path: workspace sizes of the reference geometry (one workgroup per key split and KV head, the fp16
+    path's partial layout), and refusals before any launch (D, KVH, rows, a V pool, pools of 2 GiB,
     rows past the pool)."""
     host = load_host()
     lib = host.lib()
@@ -145,6 +145,25 @@ def test_record_entry_points_check_their_arguments():
     assert lib.dspark_kv_write_rec(fake, fake, 512, fake, None, 10, 4, 300, 40, None) == 1001
     assert lib.dspark_kv_write_rec(fake, fake, 256, fake, None, 10, 4, 0, 1, None) == 1001   # row < KVH * 128
     assert lib.dspark_kv_write_rec(None, fake, 512, fake, None, 10, 4, 0, 1, None) == 1001
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 12, 16])
+def test_record_splits_follow_the_range_alone(M):
+    """The record attention's own split counts: a split's running max is where its rows' P are rounded, so the outputs' last
+    bits hang on the count, and it is the same for every number of tokens: a page per split up to 96 pages, then two or
+    more (256 splits at most)."""
+    host = load_host()
+    lib = host.lib()
+    for pages in (1, 2, 32, 64, 65, 95, 96, 97, 129, 193, 256, 257, 511, 512, 513, 1025, 2048, 4096):
+        args = host.AttnArgs()
+        args.M, args.QH, args.KVH, args.D, args.a, args.causal = M, 16, 4, 128, 32 * pages - M, 1
+        if args.a < 0:
+            continue
+        most = pages if pages <= 96 else min(256, (pages + 1) // 2)
+        per = (pages + most - 1) // most
+        slots = 4 * ((pages + per - 1) // per) * 16 * ((4 * M + 15) // 16)   # heads x splits x padded rows
+        want = sum((slots * b + 255) // 256 * 256 for b in (128 * 4, 8))
+        assert lib.dspark_verify_attention_rec_workspace(ctypes.byref(args)) == want, (pages, M)
 
 
 @pytest.mark.parametrize("base,pairs,D", [(1e6, 32, 128), (1e4, 64, 128), (1e6, 32, 64), (1e4, 16, 64)])
