@@ -114,7 +114,9 @@ struct QkRopeBatch {
   int n;
 };
 int qkrope_batch_launch(const QkRopeBatch& b, hipStream_t s);
-// The same for whole prompts: K/V rows only (no q16, no records), positions from the State's context, page by page.
+// The same for whole prompts of up to KVROPE_PAGES_MAX positions: K/V rows only (no q16, no records), positions from the
+// State's context, page by page.
+constexpr int KVROPE_PAGES_MAX = 65000 * DSPARK_PAGE_TOKENS;
 int kvrope_pages_launch(const QkRopeBatch& b, hipStream_t s);
 
 struct MarkovParams {

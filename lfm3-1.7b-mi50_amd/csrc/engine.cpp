@@ -513,6 +513,7 @@ int enqueue_context(dspark_engine* e, const _Float16* x_fc, bool x_op, hipStream
 
 // The context projection of n prompt positions at once, x_fc row-major [n][n_taps * H]: the same four steps as
 // enqueue_context, each one launch over every position, its GEMMs (planned by project_wide_plan) on many-token tiles (gemm_wide.hip).
+// fp16 rings are written page by page; records (and more pages than that kernel's grid takes) row by row.
 constexpr int PROJ_BANDS = 2;  // proj_y holds tap_rows x PROJ_BANDS x H: fewer positions may take more bands
 bool project_wide_plan(dspark_engine* e, int n, GemmWideParams* fc, GemmWideParams* ckv) {
   const dspark_model_desc& d = e->d;
@@ -544,12 +545,13 @@ int project_wide(dspark_engine* e, const _Float16* x_fc, int n, GemmWideParams f
   p.H = H;
   CK(resnorm_launch(p, n, 1, s));
   CK(gemm_of(ckv, e->proj_x, e->ckv_w, e->ckv_s));
+  const bool by_page = d.kv_format == 0 && n <= KVROPE_PAGES_MAX;
   for (int j0 = 0; j0 < d.draft_layers; j0 += QKROPE_BATCH) {
     QkRopeBatch b = {};
     b.n = std::min(QKROPE_BATCH, d.draft_layers - j0);
     for (int j = 0; j < b.n; ++j)
       b.l[j] = qk_params(e, e->DL[j0 + j], e->proj_y + (size_t)(j0 + j) * kvrow, rows, false, true, n);
-    CK(kvrope_pages_launch(b, s));
+    CK(by_page ? kvrope_pages_launch(b, s) : qkrope_batch_launch(b, s));
   }
   return 0;
 }

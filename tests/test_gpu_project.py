@@ -4,12 +4,14 @@ and group scales, at position counts around the tiles' edges, against fp64 from 
 
 Bar: the ring holds fp16 of values whose inputs the GPU and the check round to fp16 at the same points (the captured taps,
 the hidden norm's output), so a value differs by its own rounding and by what last-bit flips of those inputs carry
-through a dot product: two fp16 steps at the largest magnitude, the bar of the blockwise projection's test."""
+through a dot product: two fp16 steps at the largest magnitude, the bar of the blockwise projection's test. A record holds
+a row of K or V in steps of its largest magnitude / 127: half a step more."""
 import numpy as np
 import pytest
 
 from conftest import load_host, rope_numpy
-from test_gpu_engine import REF_SMALL, SMALL, make_weights
+from test_gpu_engine import REF_REC, REF_SMALL, SMALL, make_weights
+from test_gpu_fullsize import ring_rows
 from test_gpu_launch import ulp16
 
 pytestmark = pytest.mark.gpu
@@ -25,6 +27,11 @@ WIDE_GROUPS = dict(WIDE, weight_format=1, n_taps=3, tap_layer=[0, 1, 2])
 CASES = [(NARROW, n, first) for n, first in ((9, 0), (63, 5), (64, 31), (65, 7), (128, 0), (200, 500), (700, 330))]
 CASES += [(GROUPS, n, 33) for n in (10, 64, 129, 511)]
 CASES += [(WIDE, 1537, 700), (WIDE_GROUPS, 1537, 1), (WIDE_GROUPS, 1600, 0)]
+# int8 K/V records: blocks of 9, the two position counts around a block, page edges, 64- and 128-token tiles
+RECORDS = dict(REF_REC, draft_window=700, ring_positions=1024)
+RECORDS_ROWS = dict(RECORDS, weight_format=0)
+CASES += [(RECORDS, n, first) for n, first in ((9, 3), (10, 0), (31, 1), (33, 31), (64, 32), (600, 77))]
+CASES += [(RECORDS_ROWS, 10, 23), (RECORDS_ROWS, 417, 5)]
 
 
 @pytest.mark.parametrize("geom,n,first", CASES)
@@ -50,6 +57,7 @@ def test_many_positions(geom, n, first):
     kv = rnd.gemm(x, *W.gemm_w("ckv", desc.draft_layers * 2 * KVH * D, H)).reshape(n, desc.draft_layers, 2, KVH, D)
     rope = rnd.h2f(rope_numpy(desc.rope_base, desc.rope_pairs, D, first + n))[first:][:, None, :]
     cos, sin, half, p = rope[..., :D // 2], rope[..., D // 2:], D // 2, desc.rope_pairs
+    rec = desc.kv_format == 1
     bt = torch.from_numpy(eng.download("ring_table", np.int32))
     for j in range(desc.draft_layers):
         k = kv[:, j, 0]
@@ -57,12 +65,18 @@ def test_many_positions(geom, n, first):
         wk = k.copy()
         wk[..., :p] = k[..., :p] * cos[..., :p] - k[..., half:half + p] * sin[..., :p]
         wk[..., half:half + p] = k[..., half:half + p] * cos[..., :p] + k[..., :p] * sin[..., :p]
+        gk, gv = ring_rows(eng, desc, j, range(first, first + n))
+        kerr, verr = np.abs(gk - wk), np.abs(gv - kv[:, j, 1])
+        print(f"layer {j}: K max-abs {np.max(kerr):.2e}, V max-abs {np.max(verr):.2e}", flush=True)
+        for err, want in ((kerr, wk), (verr, kv[:, j, 1])):
+            bar = 2 * ulp16(np.max(np.abs(want)))
+            if rec:  # half a code, of a scale whose own row differs by the bar
+                bar = bar + 0.5 * (np.max(np.abs(want), -1, keepdims=True) + bar) / 127
+            assert np.all(err <= bar), np.max(err - bar)
+        if rec:
+            continue
         kp = torch.from_numpy(eng.download(f"ring.D{j}.k", np.uint16)).view(torch.float16).reshape(-1, KVH, 32, D)
         vp = torch.from_numpy(eng.download(f"ring.D{j}.v", np.uint16)).view(torch.float16).reshape(-1, KVH, D, 32)
-        gk, gv = (a.astype(np.float64) for a in host.kv_from_pages(kp, vp, range(first, first + n), bt))
-        kerr, verr = np.max(np.abs(gk - wk)), np.max(np.abs(gv - kv[:, j, 1]))
-        print(f"layer {j}: K max-abs {kerr:.2e}, V max-abs {verr:.2e}", flush=True)
-        assert kerr <= 2 * ulp16(np.max(np.abs(wk))) and verr <= 2 * ulp16(np.max(np.abs(kv[:, j, 1])))
         outside, _ = host.kv_from_pages(kp, vp, [first + n] + ([first - 1] if first else []), bt)
         assert not np.any(outside)
     eng.close()
