@@ -337,7 +337,7 @@ __global__ __launch_bounds__(256, OCC) void verify_attn_kernel(AttnParams p) {
 // (j < PPL) for page lane pl. The workgroup brings a step's pages from HBM into one slot of a RING-slot LDS ring with
 // direct-to-LDS buffer loads -- every page byte crosses HBM once -- and each wave reads its page lane's PPL pages from
 // LDS for its rows. RING - 1 steps (64 KB per CU) are in flight while one is computed:
-//   step k:  s_waitcnt (this wave's loads of step k done) ; s_barrier (everyone's) ; issue step k + RING - 1 into the
+//   step k:  s_waitcnt (this wave's loads of step k done) ; barrier (everyone's, and their LDS reads) ; issue step k + RING - 1 into the
 //            slot of step k - 1 (free: every wave finished step k - 1 before the barrier) ; compute step k.
 // The ring slots are separate LDS arrays selected by static index (the loop is unrolled by RING), which lets the
 // compiler see that reads of slot k never alias the loads in flight into the other slots, so it keeps the counted
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPW));
     else
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __builtin_amdgcn_s_barrier();
+    lds_barrier();
     if (k + RING - 1 < nsteps) issue(k + RING - 1, nxt);
     // fresh positions in this step's pages: their K / V rows into the LDS copy (stale in the pool), then a barrier
     if (fresh && p.a + p.M - 1 >= (pb + k * PPS) * PAGE && p.a < min(pe, pb + (k + 1) * PPS) * PAGE) {
@@ -481,8 +481,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
               fvh[e];
         }
       }
-      __builtin_amdgcn_s_waitcnt(LGKMCNT0_IMM);
-      __builtin_amdgcn_s_barrier();
+      lds_barrier();
     }
 #pragma unroll
     for (int j = 0; j < PPL; ++j) {
@@ -584,7 +583,7 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPW));
   else
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-  __builtin_amdgcn_s_barrier();
+  lds_barrier();
   if (fresh) {
     // The raw rows are first used here: an empty asm that rewrites them keeps the compiler from moving any use (a
     // conversion) up next to its load, where it would wait for the loads before the pages were issued.

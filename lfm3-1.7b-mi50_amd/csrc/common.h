@@ -68,9 +68,8 @@ __device__ __forceinline__ T ldg_nt(const T* p) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// s_waitcnt immediates (gfx9 encoding): vmcnt(n) with expcnt and lgkmcnt left at their maxima; lgkmcnt(0) alone.
+// s_waitcnt immediate (gfx9 encoding): vmcnt(n) with expcnt and lgkmcnt left at their maxima.
 __device__ __forceinline__ constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
-constexpr int LGKMCNT0_IMM = 0xC07F;
 
 // A ring step's hand-over: this wave's direct-to-LDS loads but the N youngest done, and its reads of the step before (whose
 // slot the loads issued next overwrite), then every wave's. The wait and barrier builtins do not order memory operations
@@ -84,7 +83,8 @@ __device__ __forceinline__ void ring_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Every wave's LDS accesses done, none moved across (loads from memory stay in flight).
+// Every wave's LDS accesses done, none moved across (loads from memory stay in flight). The barrier of every hand-over of
+// LDS between waves that is not a ring step's or a __syncthreads() (which would drain the loads).
 __device__ __forceinline__ void lds_barrier() { ring_barrier<63>(); }
 
 // Butterfly over a whole wave without the LDS unit (a shuffle there costs about 100 cycles a level): level by level each

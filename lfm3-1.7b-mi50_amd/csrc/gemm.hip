@@ -213,7 +213,6 @@ constexpr int GEMM_CPOL_NT = 2;         // buffer-op cache policy NT: each weigh
 constexpr int GEMM_CPOL_COHERENT = 16;  // buffer-op cache policy SC1: device-scope coherent store / load
 // s_waitcnt immediate: vmcnt(n) (6 bits, split low 4 / high 2), other counters left unconstrained
 #define GEMM_VMCNT(n) ((((n) & 15) | (((n) >> 4) << 14)) | 0x0F70)
-#define GEMM_LGKMCNT0 0xC07F  // lgkmcnt(0), vmcnt and expcnt unconstrained
 constexpr int GEMM_FIXUP_BATCH = 8;     // split partials loaded per batch by the last split
 
 // Weight loads go in batches of CPB chunks (64 columns: 16 B per lane int8, 32 B fp16), two batches in registers.
@@ -333,7 +332,7 @@ __global__ __launch_bounds__(512) void gemm_kernel(GemmParams p) {
   u32x4 wa[CPB][WV], wb[CPB][WV];
   for (int ph = c0; ph < c1; ph += PH) {
     const int pc = min(PH, c1 - ph), pe = ph + pc;
-    if (ph != c0) __syncthreads();  // every wave is done reading the previous phase
+    if (ph != c0) lds_barrier();  // every wave is done reading the previous phase
     if (xreg) {
       // One load = 8 tokens x one 64-column chunk: lane l reads token 8 (k % 2TB) + l / 8, 16 B at column
       // 64 j + 8 (l % 8) of chunk j = k / 2TB, so a load covers 8 whole 128-byte lines. The wave's X loads (at most
@@ -360,8 +359,7 @@ __global__ __launch_bounds__(512) void gemm_kernel(GemmParams p) {
         if (k < ninstr && t < p.M)
           xs[(((t >> 4) * pc + j) * 2 + hq) * 64 + (((t & 15) + 16 * gq) ^ (4 * gq + 2 * hq))] = xr[i];
       }
-      __builtin_amdgcn_s_waitcnt(GEMM_LGKMCNT0);  // this wave's LDS writes (the weights stay in flight)
-      __builtin_amdgcn_s_barrier();
+      lds_barrier();  // (the weights stay in flight)
     } else {
     // Issue order: this wave's X rows, then the phase's first two weight batches; the counted wait below then covers
     // X (the oldest loads) and leaves the weights in flight.
@@ -384,7 +382,7 @@ __global__ __launch_bounds__(512) void gemm_kernel(GemmParams p) {
     } else {
       __builtin_amdgcn_s_waitcnt(GEMM_VMCNT(CPB * WV));
     }
-    __builtin_amdgcn_s_barrier();
+    lds_barrier();
     }
     for (int cb = ph; cb < pe; cb += 2 * CPB) {
       compute(wa, cb, ph, pc);
@@ -833,8 +831,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
     if constexpr (GS) gscale_load<CPW>(p, rgs, gsr, c0, c1, gvo);  // older than X: covered by the wait below
     stage(0, min(tbp, TB));
     load(w, c0);
-    __builtin_amdgcn_s_waitcnt(GEMM_VMCNT(CPW * WV));
-    __builtin_amdgcn_s_barrier();
+    ring_barrier<CPW * WV>();  // X^T is in LDS, the weights in flight
     if constexpr (X8 == 1) {
       // x quantized where it lies, each chunk once in the workgroup (lane (n, g): token n's piece g): the products below
       // then read codes and scales as the norm would have left them.
@@ -845,8 +842,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
         xr[0] = lo;
         xr[64] = hi;
       }
-      __builtin_amdgcn_s_waitcnt(GEMM_LGKMCNT0);  // (the weights stay in flight)
-      __builtin_amdgcn_s_barrier();
+      lds_barrier();  // (the weights stay in flight)
     }
     if constexpr (X8) {  // one token block, X^T of the band in LDS at once, as below
       for (int cb = c0; cb < c1; cb += CPW) {
@@ -919,8 +915,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
           if (t0 > 0) {
             __syncthreads();  // every wave is done with the previous pass's X^T
             stage(t0, min(PT, TB - t0));
-            __builtin_amdgcn_s_waitcnt(0);
-            __builtin_amdgcn_s_barrier();
+            ring_barrier<0>();
           }
 #pragma unroll
           for (int i = 0; i < CPW; ++i) {
