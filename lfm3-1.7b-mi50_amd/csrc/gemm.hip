@@ -1655,6 +1655,15 @@ static bool gemm_plan_sliced(int N, int K, int tb, bool i8, int wpg_req, bool xo
       KW = std::min(8, std::max(4, (gbc + 7) / 8));
       xd = true;
     }
+    // KW ranges rounded up to whole groups where that saves a batch of 8 chunks, else the largest count of ranges that are
+    // even by themselves; never an idle one (its waves take part in every barrier and in the sum). 8 tokens, rounded / even:
+    // 8192 x 1792 8, 8, 8, 4 chunks against 10, 10, 8: 7.8 / 8.8 us; 8192 x 2304 10, 10, 10, 6 against 3 x 12: 11.1 / 10.6;
+    // 9984 x 640 4, 4, 2, 0 against 4, 4, 2: 8.3 / 7.3.
+    const int round = gemm_range_chunks(gbc, KW, true);
+    int even = KW;
+    while (even > 1 && ((gbc + even - 1) / even) % 2) --even;
+    const int per = ((gbc + even - 1) / even + 7) / 8 <= (round + 7) / 8 ? (gbc + even - 1) / even : round;
+    KW = (gbc + per - 1) / per;
   }
   // X^T through LDS: all token blocks at once when they fit 64 KB, else one token block per pass, each pass's X^T
   // within 64 KB and each range within one 8-chunk batch (its weights stay in registers)

@@ -1,0 +1,43 @@
+"""The GEMMs' plans (which kernel, tiles and shares of K a shape takes), without a GPU."""
+import ctypes
+
+import pytest
+
+from conftest import load_host
+
+FIELDS = ["ksplit", "wpg", "cpb", "kw", "xd", "bands", "stream", "few"]
+
+
+class Plan(ctypes.Structure):
+    """GemmPlan (dspark_internal.h)."""
+    _fields_ = [(f, ctypes.c_int) for f in FIELDS]
+
+
+def plan(M, N, K, i8=True, split=False, wpg=0, xop=False, bands=1, gs=False, rows=True, x8=False):
+    """rows: x and w row-major on 16-byte boundaries."""
+    p = Plan(1, 1, 4, 0, 0, 1, 0, 0)
+    host = load_host()
+    f = getattr(host.lib(), "_ZN6dspark9gemm_planEiiibbPNS_8GemmPlanEibibbb")
+    f.argtypes = [ctypes.c_int] * 3 + [ctypes.c_bool] * 2 + [ctypes.POINTER(Plan), ctypes.c_int, ctypes.c_bool, ctypes.c_int] + \
+        [ctypes.c_bool] * 3
+    f.restype = None
+    f(M, N, K, i8, split, ctypes.byref(p), wpg, xop, bands, gs, rows, x8)
+    return p
+
+
+@pytest.mark.parametrize("x8", [False, True])
+@pytest.mark.parametrize("rows,xop,wpg,bands", [(True, False, 0, 1), (False, False, 0, 1), (False, True, 0, 1),
+                                                (False, True, 0, 2), (False, True, 3, 1)])
+def test_group_scale_ranges(rows, xop, wpg, bands, x8):
+    """Ranges of K under group scales hold whole groups (two 64-column chunks), and none is empty: an idle range's waves
+    would take part in every barrier and in the sum."""
+    for N in (48, 512, 2048, 3072, 4096, 6144, 8208, 9984, 16464, 65520):
+        for K in range(128, 8193, 128):
+            for M in (1, 4, 9, 16):
+                p = plan(M, N, K, wpg=wpg, xop=xop, bands=bands, gs=True, rows=rows, x8=x8)
+                if p.kw == 0 or p.few:
+                    continue
+                band = (K // 64 + p.bands - 1) // p.bands
+                per = (band + p.kw - 1) // p.kw
+                per += per & 1
+                assert (p.bands == 1 or band % 2 == 0) and (p.kw - 1) * per < band, (M, N, K, p.kw, per, band)
