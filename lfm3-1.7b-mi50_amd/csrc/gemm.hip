@@ -1009,6 +1009,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
 // GS (one token block): per-128-column group scales, one group per step: the step's products go to a fresh accumulator
 // that is scaled and added, as in the K-sliced kernel; its rows' scales ride in the slot, one copy per wave.
 constexpr int GEMM_STREAM_WGS = 256;  // one workgroup per CU (the ring)
+constexpr int GEMM_STREAM_SLOTS = 8;  // the ring of up to two token blocks and tiles of 4 strips
 template <int TB, int WB, int RS, int NW, int SLOTS, bool GS>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p) {
   constexpr int TG = NW / RS, TBW = (TB + TG - 1) / TG;         // token groups; token blocks of a wave
@@ -1511,7 +1512,7 @@ static void launch_stream_tb(const GemmParams& p, hipStream_t s) {
       return;
     }
   }
-  launch_stream_as<TB, WB, 4, TB == 1 ? 4 : 8, TB <= 2 ? 8 : 4, GS>(p, s);
+  launch_stream_as<TB, WB, 4, TB == 1 ? 4 : 8, TB <= 2 ? GEMM_STREAM_SLOTS : 4, GS>(p, s);
 }
 template <bool I8>
 static void launch_stream(const GemmParams& p, hipStream_t s) {
@@ -1701,6 +1702,11 @@ static bool gemm_plan_stream(int M, int N, int K, bool i8, bool split, bool gs, 
   const int wb = i8 ? 1 : 2, strips = N / 16, steps = K * wb / 128;
   if ((size_t)K * wb % 128 || (size_t)N * K * wb >= (size_t)1 << 31 || (size_t)M * K * 2 >= (size_t)1 << 31) return false;
   if (gs && M > 16) return false;
+  // Group scales, more tiles than workgroups and K up to 2048 (whose X^T the K-sliced kernel holds in LDS): only where a tile
+  // is whole turns of the ring, so that tiles follow each other in it. Otherwise every tile is a workgroup that fills the
+  // ring anew (8 tokens, K-sliced / streamed: 65536 x 512 10.1 / 15.8 us, 20480 x 1536 10.8 / 13.5, 128000 x 1792 58 / 60;
+  // past 2048 65536 x 2304 even, x 4224 2.5 times faster streamed).
+  if (gs && (strips + 3) / 4 > GEMM_STREAM_WGS && K <= 2048 && steps % GEMM_STREAM_SLOTS) return false;
   const auto per_cu = [&](int rs) { return rs * ((strips + rs * GEMM_STREAM_WGS - 1) / (rs * GEMM_STREAM_WGS)); };
   const int rs = i8 && !gs && per_cu(8) <= per_cu(4) ? 8 : 4;
   const int tiles = (strips + rs - 1) / rs;

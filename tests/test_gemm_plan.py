@@ -41,3 +41,14 @@ def test_group_scale_ranges(rows, xop, wpg, bands, x8):
                 per = (band + p.kw - 1) // p.kw
                 per += per & 1
                 assert (p.bands == 1 or band % 2 == 0) and (p.kw - 1) * per < band, (M, N, K, p.kw, per, band)
+
+
+@pytest.mark.parametrize("M", [1, 8, 16])
+def test_streamed_group_scales(M):
+    """Row-major group scales over more tiles (64 rows) than workgroups: streamed where a tile is whole turns of the 8-slot
+    ring (128 columns a step), or K is past what the K-sliced kernel holds in LDS."""
+    for N in (16400, 20480, 65536, 128000):
+        for K in range(128, 4609, 128):
+            assert bool(plan(M, N, K, gs=True).stream) == (K % 1024 == 0 or K > 2048), (N, K)
+    for K in (256, 640, 2048, 2304):
+        assert plan(M, 16384, K, gs=True).stream == 4
