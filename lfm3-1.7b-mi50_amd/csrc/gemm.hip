@@ -1682,8 +1682,12 @@ static bool gemm_plan_sliced(int N, int K, int tb, bool i8, int wpg_req, bool xo
 
 // Few-row plans (row-major operands on 16-byte boundaries): one group of 8 rows per workgroup while those are at most one
 // per CU, else two.
-static bool gemm_plan_few(int M, int N, int K, bool gs, GemmPlan* pl) {
+// fp16 x with two groups to a workgroup only up to K 1024 or 3 tokens: past both, every wave's own x outweighs its 8 rows of
+// weights, and the K-sliced kernel's 16-row strips halve it (3072 rows, K-sliced / few-row: K 4096 7.4 / 7.2 us at 3 tokens,
+// 7.9 / 9.9 at 9, 9.1 / 12.5 at 16; K 1024 4.8 / 4.3 at 8).
+static bool gemm_plan_few(int M, int N, int K, bool gs, bool x8, GemmPlan* pl) {
   if (!gs || M > 16 || K % 128 || N > 16 * GEMM_STREAM_WGS) return false;
+  if (!x8 && N > 8 * GEMM_STREAM_WGS && K > 1024 && M > 3) return false;
   *pl = GemmPlan{};
   pl->few = 1;
   pl->wpg = N > 8 * GEMM_STREAM_WGS ? 2 : 1;
@@ -1723,7 +1727,7 @@ static bool gemm_plan_stream(int M, int N, int K, bool i8, bool split, bool gs, 
 void gemm_plan(int M, int N, int K, bool i8, bool split, GemmPlan* pl, int wpg_req, bool xop, int max_bands, bool gs,
                bool stream, bool x8) {
   const int strips = N / 16, chunks = K / 64, tb = (M + 15) / 16;
-  if (stream && gemm_plan_few(M, N, K, gs, pl)) return;
+  if (stream && gemm_plan_few(M, N, K, gs, x8, pl)) return;
   if (stream && !x8 && gemm_plan_stream(M, N, K, i8, split, gs, pl)) return;
   if (gemm_plan_sliced(N, K, tb, i8, wpg_req, xop, max_bands, pl, gs)) return;
   pl->kw = 0;

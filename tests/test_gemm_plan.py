@@ -52,3 +52,17 @@ def test_streamed_group_scales(M):
             assert bool(plan(M, N, K, gs=True).stream) == (K % 1024 == 0 or K > 2048), (N, K)
     for K in (256, 640, 2048, 2304):
         assert plan(M, 16384, K, gs=True).stream == 4
+
+
+def test_few_rows():
+    """Row-major group scales up to 4096 rows: groups of 8 rows, two to a workgroup past 2048 rows; fp16 x then only up to K
+    1024 or 3 tokens."""
+    for M in range(1, 17):
+        for N in (16, 512, 2048, 2064, 3072, 4096, 4112):
+            for K in range(128, 8193, 128):
+                two = N > 2048
+                for x8 in (False, True):
+                    want = N <= 4096 and (x8 or not two or K <= 1024 or M <= 3)
+                    p = plan(M, N, K, gs=True, x8=x8)
+                    assert bool(p.few) == want, (M, N, K, x8)
+                    assert not want or p.wpg == 1 + two and p.kw == min(16 // p.wpg, K // 128)

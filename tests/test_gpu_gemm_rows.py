@@ -80,7 +80,7 @@ def test_head_rows(M, N, K, off):
 
 GROUPS = [(1, 16, 128), (8, 48, 256), (9, 2064, 640), (16, 4096, 1920), (7, 2048, 2304), (16, 2048, 7680), (9, 4112, 4096),
           (16, 8256, 1024), (3, 15360, 2048), (16, 16464, 384), (9, 9984, 640), (8, 8192, 1792),
-          (8, 20480, 768), (5, 17424, 1024)]
+          (8, 20480, 768), (5, 17424, 1024), (3, 2064, 1152), (4, 2064, 1152), (16, 4096, 1152)]
 
 
 @pytest.mark.parametrize("x8", [False, True])
