@@ -639,8 +639,9 @@ __global__ __launch_bounds__(1024) void markov_chain_kernel(MarkovParams p) {
       break;
     }
     if (tid == 0) st->tokens[j] = prev;
-    // the thread's largest value and its first row (rows in rising order: a later one has to be larger)
-    uint32_t bo = 0, br = 0xffffffffu;
+    // the thread's largest value and its first row (rows in rising order: a later one has to be larger; the first live row
+    // stands for a NaN of all ones too, whose order is 0)
+    uint32_t bo = 0, br = live(0) ? (uint32_t)r0 : 0xffffffffu;
 #pragma unroll
     for (int i = 0; i < CHAIN_QUADS; ++i)
       if (live(i)) {
