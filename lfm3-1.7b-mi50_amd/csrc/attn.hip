@@ -394,7 +394,11 @@ __global__ __launch_bounds__(MAXW * 64) void verify_attn_lds_kernel(AttnParams p
   const int wave = __builtin_amdgcn_readfirstlane(TID >> 6);
   const int NRB = p.nrb, NRG = p.nrg, NW = NRG * PL;
   static_assert(PL <= 4, "page lanes by comparison");
-  const int pl = (PL > 1 && wave >= NRG) + (PL > 2 && wave >= 2 * NRG) + (PL > 3 && wave >= 3 * NRG);
+  int pl = (PL > 1 && wave >= NRG) + (PL > 2 && wave >= 2 * NRG) + (PL > 3 && wave >= 3 * NRG);
+  // One page lane: a 0 the compiler does not know. With every LDS address a constant it makes each one past the 64 KB that a
+  // read's offset reaches anew, between the reads, instead of one base per page (D = 128, two layers of 131072 keys: 33 tokens
+  // 153.7 / 143.2 us, 48 tokens 177.3 / 165.7, 64 tokens 202.3 / 190.8).
+  if constexpr (PL == 1) asm("" : "+s"(pl));
   const int rg = wave - pl * NRG;
   const int h = WG_Y, split = WG_X;
   const int R = NRB * 16;
