@@ -30,6 +30,14 @@ CASES += [(WIDE, 1537, 700), (WIDE_GROUPS, 1537, 1), (WIDE_GROUPS, 1600, 0)]
 # int8 K/V records: blocks of 9, the two position counts around a block, page edges, 64- and 128-token tiles
 RECORDS = dict(REF_REC, draft_window=700, ring_positions=1024)
 RECORDS_ROWS = dict(RECORDS, weight_format=0)
+# fc in 16, 8 and 4 bands (128 chunks of K; one, two and four token tiles of 64), and in 4 of 15 chunks (16 and a short last
+# one with group scales)
+BANDS = dict(WIDE, n_taps=4, tap_layer=[0, 1, 2, 3])
+BANDS_GROUPS = dict(BANDS, weight_format=1)
+UNEVEN = dict(WIDE, hidden=1280, q_heads=20, kv_heads=5, n_taps=3, tap_layer=[0, 1, 2])
+UNEVEN_GROUPS = dict(UNEVEN, weight_format=1)
+CASES += [(geom, n, 9) for geom in (BANDS, BANDS_GROUPS) for n in (17, 64, 65, 200)]
+CASES += [(geom, n, 31) for geom in (UNEVEN, UNEVEN_GROUPS) for n in (10, 40)]
 CASES += [(RECORDS, n, first) for n, first in ((9, 3), (10, 0), (31, 1), (33, 31), (64, 32), (600, 77))]
 CASES += [(RECORDS_ROWS, 10, 23), (RECORDS_ROWS, 417, 5)]
 
@@ -46,6 +54,12 @@ def test_many_positions(geom, n, first):
     W = rnd.Weights(desc, make_weights(eng, desc, 7))
     rng = np.random.default_rng(n)
     taps = rng.standard_normal((desc.n_taps, n, H)).astype(np.float16)
+    rec = desc.kv_format == 1
+    names = ["rec"] if rec else ["k", "v"]
+    before = {}
+    for name in (f"ring.D{j}.{x}" for j in range(desc.draft_layers) for x in names):  # any bits: no slot starts as zeros
+        before[name] = rng.integers(0, 1 << 16, eng.tensor(name)[1] // 2).astype(np.uint16)
+        eng.upload(name, before[name])
     for slot in range(desc.n_taps):
         eng.capture_tap(slot, torch.from_numpy(taps[slot]).cuda(), first, first)
     eng.project_prompt(first, first + n)
@@ -57,8 +71,7 @@ def test_many_positions(geom, n, first):
     kv = rnd.gemm(x, *W.gemm_w("ckv", desc.draft_layers * 2 * KVH * D, H)).reshape(n, desc.draft_layers, 2, KVH, D)
     rope = rnd.h2f(rope_numpy(desc.rope_base, desc.rope_pairs, D, first + n))[first:][:, None, :]
     cos, sin, half, p = rope[..., :D // 2], rope[..., D // 2:], D // 2, desc.rope_pairs
-    rec = desc.kv_format == 1
-    bt = torch.from_numpy(eng.download("ring_table", np.int32))
+    bt = eng.download("ring_table", np.int32)
     for j in range(desc.draft_layers):
         k = kv[:, j, 0]
         k = k / np.sqrt((k * k).mean(-1, keepdims=True) + desc.eps) * W.f16(f"D{j}.k_norm")
@@ -73,10 +86,21 @@ def test_many_positions(geom, n, first):
             if rec:  # half a code, of a scale whose own row differs by the bar
                 bar = bar + 0.5 * (np.max(np.abs(want), -1, keepdims=True) + bar) / 127
             assert np.all(err <= bar), np.max(err - bar)
-        if rec:
-            continue
-        kp = torch.from_numpy(eng.download(f"ring.D{j}.k", np.uint16)).view(torch.float16).reshape(-1, KVH, 32, D)
-        vp = torch.from_numpy(eng.download(f"ring.D{j}.v", np.uint16)).view(torch.float16).reshape(-1, KVH, D, 32)
-        outside, _ = host.kv_from_pages(kp, vp, [first + n] + ([first - 1] if first else []), bt)
-        assert not np.any(outside)
+        # every slot of the ring outside [first, first + n) holds the bits it held
+        at = np.arange(first, first + n)
+        pages, slots = bt[at // 32], at % 32
+        for x in names:
+            now, was = eng.download(f"ring.D{j}.{x}", np.uint16), before[f"ring.D{j}.{x}"]
+            if rec:
+                now, was = (b.view(np.uint8).reshape(-1, 32, KVH * 264) for b in (now, was))
+                now[pages, slots] = was[pages, slots] = 0
+            elif x == "k":  # [page][head][keys in operand order][dims]
+                index = np.asarray(host.k_page_index(D))
+                now, was = (b.reshape(-1, KVH, 32 * D) for b in (now, was))
+                for pg, sl in zip(pages, slots):
+                    now[pg][:, index[sl]] = was[pg][:, index[sl]] = 0
+            else:  # [page][head][dims][keys]
+                now, was = (b.reshape(-1, KVH, D, 32) for b in (now, was))
+                now[pages, :, :, slots] = was[pages, :, :, slots] = 0
+            assert np.array_equal(now, was), x
     eng.close()
