@@ -251,7 +251,7 @@ struct GemmParams {
   const void* w;            // [N][K] biased int8 or fp16
   const _Float16* scale;    // [N] or nullptr
   const _Float16* gscale;   // or [K / 128][N]: one fp16 scale per (128-column group, row), the reference's per-128
-                            // format (internal/weights/quant.go:66-104); K-sliced plans with one token block only
+                            // format (internal/weights/quant.go:66-104); one token block: K-sliced, streamed and few-row plans
   const float* xsc;         // x8 == 2
   int M, N, K;
   int xop;                  // > 0: x in operand order (xop_elem) with xop >= ceil(M / 16) token blocks; 0: row-major

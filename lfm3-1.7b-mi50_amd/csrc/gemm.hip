@@ -496,10 +496,11 @@ __device__ __forceinline__ void gscale_products(f32x4& acc, const u32x2 (&gsr)[C
 // piece: lane (g, n) gives row n's / token n's columns 16 p + 4 g .. + 3 of piece p. The weight tiles of an int8-x
 // engine are laid out for it (gemm_tile_kernel, x8: byte b of lane (g, n) is column 16 (b / 4) + 4 g + b % 4 of the
 // 64-column chunk, so a[p / 2] halves 4 (p % 2) .. + 3 are piece p's four weights); row-major weights (the C ABI) are
-// brought to the same order (x8_transpose4). Codes are integer-valued halves, so each product is the piece's exact integer dot
-// (|dot| <= 16 * 127 * 127 < 2^24). p.x8 = 1: x is fp16 and each piece is quantized by the four lanes that hold it, as
-// x_fill does (883-904): s = max(max|x| / 127, 1e-20), codes rint(x * rcp(s)); p.x8 = 2: x holds the codes (the norm
-// kernel's output) and p.xsc the scales [token][K / 16].
+// brought to the same order (x8_transpose4). Codes are integer-valued halves, so each product is the piece's exact
+// integer dot (|dot| <= 16 * 127 * 127 < 2^24). p.x8 = 1: x is fp16 and each piece is quantized by the one lane that loads
+// it whole (X per wave: every wave its own operands; X^T in LDS: once in the workgroup, where it lies), as x_fill does
+// (883-904): s = max(max|x| / 127, 1e-20), codes rint(x * rcp(s)); p.x8 = 2: x holds the codes (the norm kernel's output)
+// and p.xsc the scales [token][K / 16].
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4 mfma16x16x16(half4v a, half4v b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
@@ -614,8 +615,8 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
   static_assert(!ONEB || (XD && MAXT > 512), "the one-batch form is the 1024-thread X-per-wave kernel's");
   // The stop flag is loaded first and tested once the data loads are in flight and the products computed (before
   // anything is stored), so its latency overlaps theirs; a stopped round writes nothing.
-  // The prologue up to the first weight load is on every launch's critical path (a round is a chain of some two hundred
-  // launches, half of them this kernel): no integer division, the arguments' first lines in one round trip, and buffer loads
+  // The prologue up to the first weight load is on every launch's critical path (a round is a chain of 154 launches in the
+  // 16-layer configuration, 219 in the reference geometry, a third to half of them this kernel): no integer division, the arguments' first lines in one round trip, and buffer loads
   // whose chunk offset is one scalar. (With divisions by the plan's numbers and 64-bit addresses per chunk it was 420
   // instructions, about 0.8 us a launch: 16-layer rounds 1087 -> 1057 us, reference geometry 1389 -> 1372.)
   asm volatile("" ::"s"(p.st), "s"(p.wpg), "s"(p.conv_ring));
@@ -1002,7 +1003,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
 // step issues the same loads and the waits are counted. Tiles beyond one per workgroup follow each other in the same
 // stream (no new fill of the ring). K split over workgroups (p.ksplit): the partials and the last arrival's sum as in
 // gemm_kernel.
-// Bound by HBM (one token block: 5.1 TB/s of weights at 65536 x 2048) and, with more tokens, by the LDS reads of x that each
+// Bound by HBM (one token block: 5.1 TB/s of weights at 65536 x 2048, three sets of them in turn) and, with more tokens, by the LDS reads of x that each
 // strip's wave makes. Measured against the K-sliced and split kernels on row-major operands: 16384 x 2048 and 2048 x 8192
 // at 16 tokens 12.2 and 11.2 -> 9.7 and 9.6 us, at 64 tokens 21.5 and 21.1 -> 12 and 14; 128000 x 2048 at 16 tokens with its
 // argmax 68.3 -> 58.6, at 64 118 -> 84; fp16 16384 x 2048 at 64 tokens 34.4 -> 19.7.
@@ -1506,7 +1507,7 @@ static void launch_stream_as(const GemmParams& p, hipStream_t s) {
 }
 template <int TB, int WB, bool GS>
 static void launch_stream_tb(const GemmParams& p, hipStream_t s) {
-  if constexpr (!GS) {
+  if constexpr (!GS && WB == 1) {  // (the plan takes tiles of 8 strips for int8 row scales only)
     if (p.stream == 8) {
       launch_stream_as<TB, WB, 8, 8, 4, false>(p, s);
       return;
