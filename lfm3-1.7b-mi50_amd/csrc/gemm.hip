@@ -1705,8 +1705,9 @@ static bool gemm_plan_few(int M, int N, int K, bool gs, bool x8, GemmPlan* pl) {
 // us, K-sliced / streamed): 128 tiles 6.8 / 7.6 at 4 tokens, 7.5 / 7.6 at 9; 192 tiles 10.2 / 8.4 at 4; 96 tiles 11.9 / 10.3 at 33;
 // 32 tiles 10.4 / 10.2 at 33 but at K 1024 5.9 / 6.9, at 64 tokens 13.8 / 10.3, 8.0 / 7.0 and, K 512, 5.6 / 5.2. Up to 128 tiles the
 // K-sliced kernel takes a strip a workgroup, at 128 two to every CU, whose ranges are one batch of 8 chunks up to K 2048: against
-// those 11 to 32 tokens need more tiles, or a K short of it (128 tiles, K 2048: 7.7 / 8.1 at 11, 8.7 / 9.2 at 17; K 1536 7.8 / 8.1 at
-// 20; K 1792 8.7 / 8.0 at 16; K 1024 8.0 / 5.9 at 16, 6.9 / 6.4 at 17). Past 2048 those ranges are two batches or more.
+// those 11 to 15 and 17 to 32 tokens need more tiles, or a K short of it (128 tiles, K 2048: 7.7 / 8.1 at 11, 8.7 / 9.2 at 17, but 8.4 /
+// 8.3 at 16, a whole token block; K 1536 7.8 / 8.1 at 20; K 1792 8.7 / 8.0 at 16; K 1024 8.0 / 5.9 at 16, 6.9 / 6.4 at 17). Past 2048
+// those ranges are two batches or more.
 static bool gemm_plan_stream(int M, int N, int K, bool i8, bool split, bool gs, GemmPlan* pl) {
   const int wb = i8 ? 1 : 2, strips = N / 16, steps = K * wb / 128;
   if ((size_t)K * wb % 128 || (size_t)N * K * wb >= (size_t)1 << 31 || (size_t)M * K * 2 >= (size_t)1 << 31) return false;
@@ -1722,7 +1723,7 @@ static bool gemm_plan_stream(int M, int N, int K, bool i8, bool split, bool gs, 
   int ks = 1;
   while (split && K > 4096 && tiles * ks * 2 <= GEMM_STREAM_WGS && steps / (2 * ks) >= 4) ks *= 2;
   const int least = GEMM_STREAM_WGS * (M <= 10 ? 6 : M <= 32 ? 4 : M <= 48 ? 3 : 0) / 8;
-  const bool one_batch = M > 10 && M <= 32 && K <= 2048 && K > (M <= 16 ? 1792 : 1024);
+  const bool one_batch = K <= 2048 && ((M > 10 && M < 16 && K > 1792) || (M > 16 && M <= 32 && K > 1024));
   if (i8 && ks == 1 && tiles < least + one_batch) return false;
   const int spk = (steps + ks - 1) / ks;
   *pl = GemmPlan{};

@@ -70,7 +70,7 @@ def test_few_rows():
 
 def test_streamed_row_scales():
     """Row-major row scales without a split of K: the fewest tiles (4 or 8 strips) that are streamed."""
-    for M, K, tiles in ((1, 2048, 192), (10, 512, 192), (11, 1792, 128), (11, 2048, 129), (16, 1024, 128), (16, 2048, 129),
+    for M, K, tiles in ((1, 2048, 192), (10, 512, 192), (11, 1792, 128), (11, 2048, 129), (15, 2048, 129), (16, 1024, 128), (16, 2048, 128),
                         (17, 1024, 128), (17, 1152, 129), (32, 2048, 129), (32, 2176, 128), (33, 2048, 96), (48, 4096, 96)):
         assert not plan(M, 64 * tiles - 64, K, split=True).stream, (M, K)
         assert plan(M, 64 * tiles, K, split=True).stream == 4 and plan(M, 64 * tiles, K, split=True).ksplit == 1, (M, K)
