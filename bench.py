@@ -366,9 +366,9 @@ def bench_c3(args, host, torch):
         "config": {"workload": "C3 (BASELINE configs[2]): M=16, FFN 2048->8192 (SiLU epilogue)->2048 int8 with per-row "
                                "fp16 scales, then 2048x16384 fp16 crop head + row argmax",
                    "algorithmic_bytes_per_step": total_bytes, "flops_per_step": flops_ffn + flops_crop},
-        "kernels": [k("up 8192x2048 int8 (gemm_kernel)", t_up, bytes_up, flops_ffn / 2),
-                    k("down 2048x8192 int8 (gemm_kernel + split-K reduce)", t_dn, bytes_dn, flops_ffn / 2),
-                    k("crop 16384x2048 fp16 + argmax (gemm_kernel<fp16> + fold)", t_crop, bytes_crop, flops_crop)],
+        "kernels": [k("up 8192x2048 int8", t_up, bytes_up, flops_ffn / 2),
+                    k("down 2048x8192 int8", t_dn, bytes_dn, flops_ffn / 2),
+                    k("crop 16384x2048 fp16 + argmax (product + fold)", t_crop, bytes_crop, flops_crop)],
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
                      "mfma_util": round((flops_ffn + flops_crop) / (t_step * 1e-3) / 1e12 / MFMA_F16_PEAK_TFLOPS, 4)},

@@ -616,7 +616,7 @@ __global__ __launch_bounds__(MAXT) void gemm_sliced_kernel(GemmParams p) {
   // The stop flag is loaded first and tested once the data loads are in flight and the products computed (before
   // anything is stored), so its latency overlaps theirs; a stopped round writes nothing.
   // The prologue up to the first weight load is on every launch's critical path (a round is a chain of 154 launches in the
-  // 16-layer configuration, 219 in the reference geometry, a third to half of them this kernel): no integer division, the arguments' first lines in one round trip, and buffer loads
+  // 16-layer configuration, 218 in the reference geometry, half of them this kernel): no integer division, the arguments' first lines in one round trip, and buffer loads
   // whose chunk offset is one scalar. (With divisions by the plan's numbers and 64-bit addresses per chunk it was 420
   // instructions, about 0.8 us a launch: 16-layer rounds 1087 -> 1057 us, reference geometry 1389 -> 1372.)
   asm volatile("" ::"s"(p.st), "s"(p.wpg), "s"(p.conv_ring));
