@@ -331,7 +331,8 @@ struct GemmWideParams {
   int n, N, K;
   int tile, bands, band_chunks;  // gemm_wide_plan: rows and tokens of a tile, shares of K and their 64-column chunks
 };
-// false: a shape this kernel does not take (N % 128, operands of 2 GiB or more)
+// false: a shape this kernel does not take (N % 128, operands above GEMM_WIDE_MAX_BYTES: 32-bit load offsets)
+constexpr int64_t GEMM_WIDE_MAX_BYTES = ((int64_t)1 << 31) - 1;
 bool gemm_wide_plan(int n, int N, int K, bool gs, int max_bands, GemmWideParams* p);
 int gemm_wide_launch(const GemmWideParams& p, hipStream_t s);
 

@@ -106,9 +106,10 @@ struct dspark_engine {
   // State per projection chunk (ctx_pos, ctx_new of the chunk)
   _Float16* tapx = nullptr;
   int tap_rows = 0, tap_from = -1;
-  // whole-prompt projection (project_wide): the GEMM outputs of up to tap_rows positions (fc's two bands, then ckv's
+  // whole-prompt projection (project_wide): the GEMM outputs of up to proj_rows positions (fc's two bands, then ckv's
   // rows) and the hidden norm's x
   float* proj_y = nullptr;
+  int proj_rows = 0;
   _Float16* proj_x = nullptr;
   dspark_state* seed_st = nullptr;
   int seed_chunks = 0;
@@ -514,11 +515,11 @@ int enqueue_context(dspark_engine* e, const _Float16* x_fc, bool x_op, hipStream
 // The context projection of n prompt positions at once, x_fc row-major [n][n_taps * H]: the same four steps as
 // enqueue_context, each one launch over every position, its GEMMs (planned by project_wide_plan) on many-token tiles (gemm_wide.hip).
 // fp16 rings are written page by page; records (and more pages than that kernel's grid takes) row by row.
-constexpr int PROJ_BANDS = 2;  // proj_y holds tap_rows x PROJ_BANDS x H: fewer positions may take more bands
+constexpr int PROJ_BANDS = 2;  // proj_y holds proj_rows x PROJ_BANDS x H: fewer positions may take more bands
 bool project_wide_plan(dspark_engine* e, int n, GemmWideParams* fc, GemmWideParams* ckv) {
   const dspark_model_desc& d = e->d;
   const bool gs = d.weight_format == 1;
-  return gemm_wide_plan(n, d.hidden, d.n_taps * d.hidden, gs, PROJ_BANDS * e->tap_rows / n, fc) &&
+  return n <= e->proj_rows && gemm_wide_plan(n, d.hidden, d.n_taps * d.hidden, gs, PROJ_BANDS * e->proj_rows / n, fc) &&
          gemm_wide_plan(n, d.draft_layers * 2 * d.kv_heads * d.head_dim, d.hidden, gs, 1, ckv);
 }
 int project_wide(dspark_engine* e, const _Float16* x_fc, int n, GemmWideParams fc, GemmWideParams ckv, hipStream_t s) {
@@ -902,9 +903,10 @@ int dspark_engine_create(const dspark_model_desc* desc, int32_t max_context, dsp
   // GEMM reads), one State per chunk of B positions
   e->tap_rows = (d.draft_window + B - 1) / B * B + B;
   e->tapx = h16("tap_x", (size_t)e->tap_rows * d.n_taps * H);
-  if (d.x_format == 0) {
-    e->proj_y = static_cast<float*>(e->alloc("", (size_t)e->tap_rows * std::max(PROJ_BANDS * H, ckv_rows) * 4, &err));
-    e->proj_x = static_cast<_Float16*>(e->alloc("", (size_t)e->tap_rows * H * 2, &err));
+  if (d.x_format == 0) {  // (no more rows than the many-token GEMM takes: taps of less than 2 GiB)
+    e->proj_rows = (int)std::min<int64_t>(e->tap_rows, GEMM_WIDE_MAX_BYTES / ((int64_t)d.n_taps * H * 2));
+    e->proj_y = static_cast<float*>(e->alloc("", (size_t)e->proj_rows * std::max(PROJ_BANDS * H, ckv_rows) * 4, &err));
+    e->proj_x = static_cast<_Float16*>(e->alloc("", (size_t)e->proj_rows * H * 2, &err));
   }
   e->seed_chunks = e->tap_rows / B;
   e->seed_st = static_cast<dspark_state*>(e->alloc("", (size_t)e->seed_chunks * sizeof(dspark_state), &err));

@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(GemmWideParams p) {
 // groups), and the bands within the caller's buffer.
 bool gemm_wide_plan(int n, int N, int K, bool gs, int max_bands, GemmWideParams* p) {
   if (n < 1 || N % 128 || K % (gs ? 128 : 64)) return false;
-  if ((size_t)n * K * 2 >= (size_t)1 << 31 || (size_t)N * K >= (size_t)1 << 31) return false;  // 32-bit load offsets
+  if ((int64_t)n * K * 2 > GEMM_WIDE_MAX_BYTES || (int64_t)N * K > GEMM_WIDE_MAX_BYTES) return false;
   const int chunks = K / 64;
   auto tiles = [&](int d) { return (N / d) * ((n + d - 1) / d); };
   p->tile = tiles(128) >= 192 ? 128 : 64;

@@ -104,3 +104,26 @@ def test_many_positions(geom, n, first):
                 now[pages, :, :, slots] = was[pages, :, :, slots] = 0
             assert np.array_equal(now, was), x
     eng.close()
+
+
+def test_long_window_memory():
+    """A drafter window beyond what the one-pass projection takes (taps of 2 GiB) holds no projection buffers for the rest
+    of it; ranges that it does take are projected as ever."""
+    import torch
+    host = load_host()
+    desc = host.model_desc(**dict(WIDE, n_taps=3, tap_layer=[0, 1, 2], draft_window=400000, ring_positions=400064))
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    eng = host.Engine(desc, 401000)
+    extra = free - torch.cuda.mem_get_info()[0] - sum(eng.tensor(n)[1] for n in eng.names())
+    print(f"case window 400000: {extra / 2**30:.2f} GiB beside the named tensors", flush=True)
+    # 174762 rows of 2 bands x 2048 fp32 and 2048 fp16, the weights' tiles, allocation granularity
+    assert extra < 174762 * 2048 * 10 + 2**30, extra
+    make_weights(eng, desc, 7)
+    rows = torch.randn((64, desc.hidden), device="cuda").to(torch.float16)
+    for slot in range(desc.n_taps):
+        eng.capture_tap(slot, rows, 390000, 390000)
+    eng.project_prompt(390000, 390064)
+    torch.cuda.synchronize()
+    assert np.any(eng.download("ring.D0.k", np.uint16))
+    eng.close()
