@@ -1681,6 +1681,12 @@ static bool gemm_plan_sliced(int N, int K, int tb, bool i8, int wpg_req, bool xo
   return true;
 }
 
+static void gemm_few_shape(int N, int K, int* few, int* wpg, int* kw) {
+  *few = 1;
+  *wpg = N > 8 * GEMM_STREAM_WGS ? 2 : 1;
+  *kw = std::min(16 / *wpg, K / 128);
+}
+
 // Few-row plans (row-major operands on 16-byte boundaries): one group of 8 rows per workgroup while those are at most one
 // per CU, else two.
 // fp16 x with two groups to a workgroup only up to K 1024 or 3 tokens: past both, every wave's own x outweighs its 8 rows of
@@ -1690,9 +1696,7 @@ static bool gemm_plan_few(int M, int N, int K, bool gs, bool x8, GemmPlan* pl) {
   if (!gs || M > 16 || K % 128 || N > 16 * GEMM_STREAM_WGS) return false;
   if (!x8 && N > 8 * GEMM_STREAM_WGS && K > 1024 && M > 3) return false;
   *pl = GemmPlan{};
-  pl->few = 1;
-  pl->wpg = N > 8 * GEMM_STREAM_WGS ? 2 : 1;
-  pl->kw = std::min(16 / pl->wpg, K / 128);
+  gemm_few_shape(N, K, &pl->few, &pl->wpg, &pl->kw);
   return true;
 }
 
@@ -1775,7 +1779,19 @@ float* gemm_ws_partials(void* ws) { return reinterpret_cast<float*>(static_cast<
 #define DSPARK_GEMM_FIXUP 1  // 0: split-K partials summed by the reduce kernel even when counters are given
 #endif
 
+// Whether the K-sliced kernel's load offsets (32 bits from a strip's weights, from x, from the scales) reach its operands.
+static bool gemm_sliced_reaches(const GemmParams& p, bool i8) {
+  const int64_t lim = (int64_t)1 << 31, K = p.K;
+  return 16 * K * (i8 ? 1 : 2) < lim && (p.xop ? 16 * p.xop : p.M) * K * 2 < lim && (!p.gscale || K / 128 * p.N * 2 < lim) &&
+         (p.x8 != 2 || (int64_t)p.M * p.xsc_row * 4 < lim);
+}
+
 int gemm_launch(GemmParams& p, bool i8, hipStream_t s) {
+  if (p.kw > 0 && !p.few && !gemm_sliced_reaches(p, i8)) {
+    // (only group scales over row-major operands get here: the few-row kernel has 64-bit addresses and needs no alignment)
+    if (!p.gscale || p.x8 == 2 || p.xop || p.tiled) return DSPARK_EINVAL;
+    gemm_few_shape(p.N, p.K, &p.few, &p.wpg, &p.kw);
+  }
   if (p.few) {
     if (!i8 || p.xop || p.yop || p.tiled || p.fuse || p.x8 > 1 || p.ysc || p.bands > 1 || p.st || p.best_part || p.M > 16 ||
         p.K % 128 || !p.gscale || p.scale || p.ksplit != 1 || p.wpg * p.kw > 16)

@@ -65,3 +65,30 @@ def case(torch, orc, M, N, K, epilogue, seed):
 ])
 def test_gemm_g128_matches_oracle(dev, orc, M, N, K, epilogue):
     case(dev, orc, M, N, K, epilogue, 40 + M + N // 16 + K // 128)
+
+
+@pytest.mark.parametrize("off", [0, 8])  # off a 16-byte boundary too: the calls the K-sliced kernel takes elsewhere
+@pytest.mark.parametrize("x8", [False, True])
+def test_columns_past_32_bit_offsets(dev, x8, off):
+    """16 rows of 2^28 columns: 4 GiB of weights, so a row's bytes lie past a 32-bit offset from its strip's. x is zero but
+    for three groups of columns, at the start, the middle and the end."""
+    torch = dev
+    host = load_host()
+    M, N, K = 2, 16, 1 << 28
+    print(f"case M={M} N={N} K={K} x8={x8} off={off}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    cols = torch.cat([torch.arange(c, c + 128, device="cuda") for c in (0, K // 2 - 128, K - 128)])
+    w = torch.randint(1, 256, (N * K + off,), generator=g, device="cuda", dtype=torch.uint8)[off:].view(N, K)
+    x = torch.zeros((M * K + off // 2,), device="cuda", dtype=torch.float16)[off // 2:].view(M, K)
+    x[:, cols] = torch.randn((M, cols.numel()), generator=g, device="cuda").to(torch.float16)
+    gs = torch.rand((K // 128, N), generator=g, device="cuda").add_(0.5).mul_(1e-3).to(torch.float16)
+    y, _ = (host.gemm_i8_g128_x8 if x8 else host.gemm_i8_g128)(x, w, gs)
+    torch.cuda.synchronize()
+    wv = (w[:, cols].double() - 128) * gs[cols // 128].double().T
+    xv = x[:, cols].double()
+    if x8:
+        p = xv.view(M, -1, 16)
+        s = (p.abs().amax(-1, keepdim=True) / 127).clamp_min(1e-20)
+        xv = ((p / s).round() * s).view(M, -1)
+    want = (xv.cpu() @ wv.cpu().T).numpy()
+    assert np.max(np.abs(y.cpu().numpy() - want)) <= 2e-3 * np.max(np.abs(want))
